@@ -164,8 +164,8 @@ void CqHandle::gemv(const uint4 *codes, const uint16_t *norms, int rows, int n_p
 void matrix_gemv(const Matrix &m, Staging &st, const uint4 *codes, const uint16_t *norms, int rows, int n_pad,
                  const float *d_x, float *d_y, int batch, hipStream_t s) {
     const float *act = d_x;
-    const bool xraw = gemv_prepass(m.group) && gemv_quad_takes_x(m.group, m.in);  // the GEMV transforms x itself
-    if (!gemv_fuses_fwht(m.group) && !xraw) {
+    const GemvPath path = gemv_path(m.group, m.in, m.dev, batch);
+    if (!path.raw) {
         st.rot.reserve(size_t(batch) * m.dev);
         if (gemv_prepass(m.group))
             launch_rot_many(d_x, nullptr, batch, batch, m.in, m.dev, m.group, m.scale, st.rot.p, s);
@@ -173,8 +173,8 @@ void matrix_gemv(const Matrix &m, Staging &st, const uint4 *codes, const uint16_
             m.transform(d_x, m.in, st.rot.p, batch, st.big, s);
         act = st.rot.p;
     }
-    const CqJob job{codes, norms, act, d_y, rows, n_pad, 0, batch};
-    launch_cq_gemv(m.geom(), job, nullptr, 0, n_pad / kRowsPerBlock, s, xraw, batch);
+    const CqJob job{codes, norms, act, d_y, rows, n_pad, 0, batch, 0};
+    launch_cq_gemv(m.geom(), job, nullptr, 0, n_pad / kRowsPerBlock, batch, path, s);
 }
 
 void CqHandle::run_device(const float *d_x, float *d_y, int batch, hipStream_t s) {
@@ -275,10 +275,10 @@ void CqHandle::linear_host(const float *x, float *y, int batch) {
     // The kernels read x straight from the pinned staging buffer where they
     // read each value once (the pre-pass or transform before the GEMV) or the
     // row is at most two windows; a GEMV that transforms a wide row in every
-    // workgroup (groups of 128 / 256) reads a device copy. y is written once
+    // workgroup (one row, groups of 128 / 256) reads a device copy. y is written once
     // per value, straight into the pinned buffer. Each host-device copy saved
     // is ~7 us of a CQ4 8192 x 8192 call (80 -> 66 us).
-    const bool x_direct = !gemv_fuses_fwht(m.group) || m.in <= 2 * kWindow;
+    const bool x_direct = m.in <= 2 * kWindow || !gemv_path(m.group, m.in, m.dev, batch).raw;
     const float *dx = st.hx.p;
     if (!x_direct) {
         st.x.reserve(nx);
@@ -439,7 +439,7 @@ void SdotHandle::linear_host(const float *x, float *y, int batch) {
 // ---------------------------------------------------------------------------
 struct Plan {
     bool sdot = false;
-    bool xraw = false;  // FP32, groups <= 64: the GEMV transforms the raw inputs itself
+    GemvPath path{};    // FP32: which GEMV runs, and from which activations
     int count = 0, batch = 1;
     std::vector<CqHandle *> cq;
     std::vector<SdotHandle *> sd;
@@ -464,12 +464,11 @@ static void plan_upload(Plan &p) {
     if (!p.sdot) {
         p.rot.reserve(size_t(p.count) * p.batch * m.dev);
         std::vector<CqJob> jobs(p.count);
-        p.xraw = gemv_prepass(m.group) && gemv_quad_takes_x(m.group, m.in);
-        const bool fused = gemv_fuses_fwht(m.group) || p.xraw;
+        p.path = gemv_path(m.group, m.in, m.dev, p.batch);
         for (int i = 0; i < p.count; ++i) {
             const Matrix &mi = p.cq[i]->m;
-            const float *act = fused ? p.xs_in[i] : p.rot.p + size_t(i) * p.batch * m.dev;
-            jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, p.ys[i], mi.out, mi.n_pad, block, p.batch};
+            const float *act = p.path.raw ? p.xs_in[i] : p.rot.p + size_t(i) * p.batch * m.dev;
+            jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, p.ys[i], mi.out, mi.n_pad, block, p.batch, 0};
             block += mi.n_pad / kRowsPerBlock;
         }
         host.assign(reinterpret_cast<uint8_t *>(jobs.data()), reinterpret_cast<uint8_t *>(jobs.data() + p.count));
@@ -572,17 +571,16 @@ static void plan_run(Plan &p, hipStream_t s, hipEvent_t gemv_start = nullptr, hi
     const Matrix &m = *p.first;
     ND_CHECK(p.sdot || (!next && !prepared), "chained run: FP32 plans neither take nor leave prepared inputs");
     ND_CHECK(!next || p.count == 1, "chained run: the producing plan must hold one matrix");
-    // x_i is [batch][in] on the device; the FP32 GEMV transforms it in-kernel
-    // unless the group exceeds one table window
+    // x_i is [batch][in] on the device
     if (!p.sdot) {
-        if (gemv_prepass(m.group) && !p.xraw)
+        if (!p.path.raw && gemv_prepass(m.group))
             launch_rot_many(nullptr, p.xptr.p, p.batch, p.count * p.batch, m.in, m.dev, m.group, m.scale, p.rot.p, s);
-        else if (!gemv_fuses_fwht(m.group) && !p.xraw)
+        else if (!p.path.raw)
             for (int i = 0; i < p.count; ++i)
                 m.transform(p.xs_in[i], m.in, p.rot.p + size_t(i) * p.batch * m.dev, p.batch, p.st.big, s);
         if (gemv_start) ND_HIP(hipEventRecord(gemv_start, s));
-        launch_cq_gemv(m.geom(), CqJob{}, reinterpret_cast<const CqJob *>(p.jobs.p), p.count, p.blocks, s, p.xraw,
-                       p.batch);
+        launch_cq_gemv(m.geom(), CqJob{}, reinterpret_cast<const CqJob *>(p.jobs.p), p.count, p.blocks, p.batch,
+                       p.path, s);
         if (gemv_stop) ND_HIP(hipEventRecord(gemv_stop, s));
         return;
     }
@@ -632,8 +630,8 @@ static void linear_many(const std::vector<CqHandle *> &hs, const float *x, float
     ND_HIP(hipMemcpyAsync(st.x.p, st.hx.p, size_t(m0.in) * sizeof(float), hipMemcpyHostToDevice, s));
     // the one transform: the shared rotated x, unless the GEMV fuses the FWHT into its table build
     const float *act = st.x.p;
-    const bool xraw = gemv_prepass(m0.group) && gemv_quad_takes_x(m0.group, m0.in);  // the GEMV transforms x itself
-    if (!gemv_fuses_fwht(m0.group) && !xraw) {
+    const GemvPath path = gemv_path(m0.group, m0.in, m0.dev, 1);
+    if (!path.raw) {
         st.rot.reserve(m0.dev);
         if (gemv_prepass(m0.group)) launch_rot_many(st.x.p, nullptr, 1, 1, m0.in, m0.dev, m0.group, m0.scale, st.rot.p, s);
         else m0.transform(st.x.p, m0.in, st.rot.p, 1, st.big, s);
@@ -649,7 +647,7 @@ static void linear_many(const std::vector<CqHandle *> &hs, const float *x, float
             runs.push_back({i, 0});
             block = 0;
         }
-        jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, st.y.p + at[i], mi.out, mi.n_pad, block, 1};
+        jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, st.y.p + at[i], mi.out, mi.n_pad, block, 1, 0};
         block += mi.n_pad / kRowsPerBlock;
         runs.back().second = block;
     }
@@ -662,7 +660,7 @@ static void linear_many(const std::vector<CqHandle *> &hs, const float *x, float
         const int first = runs[r].first;
         const int njobs = (r + 1 < runs.size() ? runs[r + 1].first : n) - first;
         launch_cq_gemv(hs[first]->m.geom(), CqJob{}, reinterpret_cast<const CqJob *>(st.jobs.p) + first, njobs,
-                       runs[r].second, s, xraw);
+                       runs[r].second, 1, path, s);
     }
     ND_HIP(hipMemcpyAsync(st.hy.p, st.y.p, at[n] * sizeof(float), hipMemcpyDeviceToHost, s));
     ND_HIP(hipStreamSynchronize(s));

@@ -169,14 +169,16 @@ __host__ __device__ inline size_t norm_index(int r, int g, int groups) {
     return (static_cast<size_t>(r / kRowsPerBlock) * groups + g) * kRowsPerBlock + r % kRowsPerBlock;
 }
 
-// Groups of 128 and 256 run the activation FWHT inside the FP32 GEMV kernel.
-// Groups up to 64 take a batched pre-pass (launch_rot_many) ahead of the
-// quarter-split GEMV; groups above one window use the generic transform pass.
+// Where the FP32 GEMV's activations are transformed. One row: groups of 128
+// and 256 inside the kernel, groups up to 64 in a pre-pass (launch_rot_many)
+// or inside the quarter-split kernel (gemv_quad_takes_x). Batches: groups up
+// to 64 as for one row, 128 and 256 in the pre-pass. Groups above one window
+// always use the generic transform pass.
 inline bool gemv_fuses_fwht(int group) { return group > 64 && group <= kWindow; }
 
 // Largest group the int8 path's one-launch prepare (FWHT + quantize in LDS) takes.
 constexpr int kSdotFusedPrepareMaxGroup = 16384;
-inline bool gemv_prepass(int group) { return group <= 64; }
+inline bool gemv_prepass(int group) { return group <= kWindow; }
 
 struct CqJob {
     const uint4 *codes;       // [n_pad / kRowsPerBlock][chunks][kRowsPerBlock]
@@ -187,6 +189,7 @@ struct CqJob {
     int n_pad;
     int block_begin;          // first workgroup index of this job
     int batch;
+    int ystride;              // floats between batch rows of y (0: rows; the one-row kernels: always rows)
 };
 
 // int8 ("SDOT") path: same code layout, activations pre-quantized.
@@ -247,17 +250,24 @@ void launch_transform(const float *x, int x_stride, float *rot, int rot_stride, 
                       int padded, int dev_positions, int group, float scale, hipStream_t s);
 
 // rot[v][0..dev) = per-group FWHT of zero-padded x for nvec vectors (groups
-// of 8 .. 64): vector v is row v % batch of x0 (xptr null) or of xptr[v / batch].
+// of 8 .. 256): vector v is row v % batch of x0 (xptr null) or of xptr[v / batch].
 void launch_rot_many(const float *x0, const float *const *xptr, int batch, int nvec, int in, int dev, int group,
                      float scale, float *rot, hipStream_t s);
 
-// njobs == 0: one job passed by value (job0); otherwise jobs_dev[0..njobs). x_raw (groups <= 64): the jobs'
-// act is the raw input [batch][in], which the GEMV transforms itself (no launch_rot_many). max_batch: the
-// largest job batch (groups <= 64 take two activation rows per pass over the codes from 2 on).
-void launch_cq_gemv(const CqGeom &g, const CqJob &job0, const CqJob *jobs_dev, int njobs, int total_blocks,
-                    hipStream_t s, bool x_raw = false, int max_batch = 1);
-// Whether callers give a group <= 64 GEMV of input width `in` the raw input instead of the pre-pass output.
-bool gemv_quad_takes_x(int group, int in);
+// How launch_cq_gemv runs jobs of `batch` rows each: on the batch kernel, and from the raw input [batch][in], which
+// the GEMV then transforms itself, or the transformed rows [batch][dev] (launch_rot_many for groups up to a window,
+// launch_transform above).
+struct GemvPath {
+    bool batched, raw;
+};
+GemvPath gemv_path(int group, int in, int dev, int batch);
+// njobs == 0: one job passed by value (job0); otherwise jobs_dev[0..njobs). The batch kernel takes every job's rows
+// from `batch`, the one-row kernels from the jobs.
+void launch_cq_gemv(const CqGeom &g, const CqJob &job0, const CqJob *jobs_dev, int njobs, int total_blocks, int batch,
+                    const GemvPath &path, hipStream_t s);
+// cq_batch.h: several activation rows per pass over the codes, products on the matrix cores.
+void launch_cq_gemv_batch(const CqGeom &g, const CqJob &job0, const CqJob *jobs_dev, int njobs, int total_blocks,
+                          int batch, bool x_raw, hipStream_t s);
 
 // Dequantize rows: y[i][0..in) = FWHT(cb[code]*norm) cropped; uses rot-sized scratch.
 // Candidate rows: output row i (< count) of a compact device-layout matrix of

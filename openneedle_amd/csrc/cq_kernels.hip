@@ -7,6 +7,7 @@
 // rebuilt per 256-position window and shared by the workgroup's 256 rows, so
 // each code costs one LDS read plus one add, in the reference's own order.
 // All files are compiled with -ffp-contract=off.
+#include "codes.h"
 #include "common.h"
 #include "wave.h"
 
@@ -519,42 +520,6 @@ struct HalfState {
     u32x4 codes[SplitShape<KIND, GROUP>::kChunks];
     uint16_t norms[SplitShape<KIND, GROUP>::kGroupsPerHalf];
 };
-
-// (x byte BYTE) & mask, one SDWA op; mask lives in an SGPR.
-template <int BYTE>
-__device__ __forceinline__ uint32_t and_byte(uint32_t mask, uint32_t x) {
-    uint32_t r;
-    if constexpr (BYTE == 0)
-        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0"
-            : "=v"(r) : "s"(mask), "v"(x));
-    else if constexpr (BYTE == 1)
-        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1"
-            : "=v"(r) : "s"(mask), "v"(x));
-    else if constexpr (BYTE == 2)
-        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2"
-            : "=v"(r) : "s"(mask), "v"(x));
-    else
-        asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3"
-            : "=v"(r) : "s"(mask), "v"(x));
-    return r;
-}
-
-// Byte offsets of the 8 table entries addressed by one code dword, in code
-// order: off[2m] from nibble 2m, off[2m+1] from nibble 2m+1.
-template <int KIND>
-__device__ __forceinline__ void slot_offsets_sdwa(uint32_t wd, uint32_t mask, uint32_t off[8]) {
-    constexpr int kRot = KIND == kNib ? 2 : 3;                      // log2(entry bytes)
-    const uint32_t X = __builtin_amdgcn_alignbit(wd, wd, 32 - kRot);  // rotate left: even nibbles
-    const uint32_t Y = __builtin_amdgcn_alignbit(wd, wd, 4 - kRot);   // rotate right: odd nibbles
-    off[0] = and_byte<0>(mask, X);
-    off[1] = and_byte<0>(mask, Y);
-    off[2] = and_byte<1>(mask, X);
-    off[3] = and_byte<1>(mask, Y);
-    off[4] = and_byte<2>(mask, X);
-    off[5] = and_byte<2>(mask, Y);
-    off[6] = and_byte<3>(mask, X);
-    off[7] = and_byte<3>(mask, Y);
-}
 
 // Byte offset of window w's activations (wave-uniform, kept scalar).
 __device__ __forceinline__ int window_offset(int w) { return __builtin_amdgcn_readfirstlane(w * kWindow * 4); }
@@ -1101,7 +1066,7 @@ __device__ __forceinline__ void quad_add_parked(const float *P, int r, float &su
 
 // XF: J.act is the raw input ([batch][in]), transformed here (quad_act_x),
 // instead of the pre-pass output ([batch][dev]).
-template <int KIND, int GROUP, int QUAD, bool XF, bool PAIRS = false>
+template <int KIND, int GROUP, int QUAD, bool XF>
 __device__ __forceinline__ void quad_rows(const CqJob &J, const CqGeom &geom, float (*T)[QuadShape<KIND, GROUP>::kFloats],
                                           float (*P)[(kQuads - 1) * QuadShape<KIND, GROUP>::kGroups * kRowsPerBlock],
                                           int blk) {
@@ -1123,69 +1088,7 @@ __device__ __forceinline__ void quad_rows(const CqJob &J, const CqGeom &geom, fl
     for (int i = 0; i < 16; ++i) lut[i] = geom.lut[i];
 
     const int stride = XF ? geom.in : dev;
-    // Two activation rows per pass over the codes (the reference pairs tokens,
-    // cq.cpp:110-152): each window's chunks are loaded once and feed both rows'
-    // tables, row b0 then row b0 + 1 (passes alternate the table and park
-    // buffers; quarter 0 adds a pass's parked groups at the next pass, before
-    // that row's next window). Per row the order of every operation is that of
-    // the one-row loop below, so the outputs are the same bits.
-    int b0 = 0;
-    for (; PAIRS && b0 + 1 < batch; b0 += 2) {
-        const __amdgpu_buffer_rsrc_t rot0 =
-            buffer_rsrc(J.act + static_cast<size_t>(b0) * stride, static_cast<uint32_t>(stride) * 4u);
-        const __amdgpu_buffer_rsrc_t rot1 =
-            buffer_rsrc(J.act + static_cast<size_t>(b0 + 1) * stride, static_cast<uint32_t>(stride) * 4u);
-        // activations of pass q = 2 w + row (past the last window: zeros)
-        auto act = [&](int q) {
-            const __amdgpu_buffer_rsrc_t &rt = (q & 1) ? rot1 : rot0;
-            if constexpr (XF) return quad_act_x<KIND, GROUP>(rt, q >> 1, r, geom.scale);
-            else return quad_act<KIND>(rt, q >> 1, r);
-        };
-        QuadState<KIND, GROUP> cur, nxt;
-        float2 xr = act(0);
-        quad_load<KIND, GROUP>(cur, codes, norms, 0, QUAD, r);
-        quad_load<KIND, GROUP>(nxt, codes, norms, 1, QUAD, r);
-        __syncthreads();  // the previous rows finished with T[0] and P
-        quad_build<KIND, GROUP>(T[0], lut, xr, QUAD, r);
-        xr = act(1);
-        __syncthreads();
-        float sum[2] = {0.0f, 0.0f}, gd = 0.0f;
-        // pass (w, row): table T[row], parked P[row]; at its start quarter 0 adds
-        // the previous pass's parked groups (the other row's, same or previous
-        // window) into that row's sum
-        auto pass = [&](auto rowc, QuadState<KIND, GROUP> &st, int w) {
-            constexpr int row = decltype(rowc)::value;
-            if (QUAD == 0 && (row == 1 || w > 0))
-                quad_add_parked<KIND, GROUP>(P[row ^ 1], r, sum[row ^ 1], row == 1 ? w : w - 1, groups);
-            quad_compute<KIND, GROUP, QUAD, row == 1>(st, T[row], P[row], r, mask, sum[row], gd, w, groups, codes,
-                                                      norms);
-            const int q = 2 * w + row;
-            quad_build<KIND, GROUP>(T[row ^ 1], lut, xr, QUAD, r);
-            xr = act(q + 2);
-            __syncthreads();
-        };
-        const int pairs = windows / 2;
-        for (int it = 0; it < pairs; ++it) {
-            const int w = 2 * it;
-            pass(std::integral_constant<int, 0>{}, cur, w);
-            pass(std::integral_constant<int, 1>{}, cur, w);
-            pass(std::integral_constant<int, 0>{}, nxt, w + 1);
-            pass(std::integral_constant<int, 1>{}, nxt, w + 1);
-        }
-        if (windows & 1) {
-            const int w = windows - 1;
-            pass(std::integral_constant<int, 0>{}, cur, w);
-            pass(std::integral_constant<int, 1>{}, cur, w);
-        }
-        if (QUAD == 0) {
-            quad_add_parked<KIND, GROUP>(P[1], r, sum[1], windows - 1, groups);
-            if (row < rows) {
-                ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0) * rows + row] = sum[0];
-                ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0 + 1) * rows + row] = sum[1];
-            }
-        }
-    }
-    for (int b = b0; b < batch; ++b) {
+    for (int b = 0; b < batch; ++b) {
         const __amdgpu_buffer_rsrc_t rot =
             buffer_rsrc(J.act + static_cast<size_t>(b) * stride, static_cast<uint32_t>(stride) * 4u);
         auto act = [&](int w) {
@@ -1266,40 +1169,7 @@ __global__ __launch_bounds__(kQuadThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
 }
 
-// The quarter GEMV for batches of two or more rows: rows in pairs over one
-// pass of the codes (each chunk loaded once for both), an odd last row alone.
-// One workgroup per CU (128 VGPRs per lane: the pair loop holds both rows'
-// state and the two tables' pipelines). 16 x CQ4 8192^2 g32: batch 2
-// 203 -> 181 us, batch 4 403 -> 356 us against one row per pass.
-template <int KIND, int GROUP, bool XF>
-__global__ __launch_bounds__(kQuadThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void cq_gemv_quad_pair_kernel(
-    CqJob job0, const CqJob *__restrict__ jobs, int njobs, CqGeom geom) {
-    using Q = QuadShape<KIND, GROUP>;
-    __shared__ __attribute__((aligned(16))) float T[2][Q::kFloats];
-    __shared__ float P[2][(kQuads - 1) * Q::kGroups * kRowsPerBlock];
-    const int blk = blockIdx.x;
-    CqJob J = job0;
-    if (njobs > 0) {
-        const ND_CONST CqJob *cj = (const ND_CONST CqJob *)(jobs);
-        const int j = find_job(cj, njobs, blk);
-        J.codes = cj[j].codes;
-        J.norms = cj[j].norms;
-        J.act = cj[j].act;
-        J.y = cj[j].y;
-        J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
-        J.block_begin = cj[j].block_begin;
-        J.batch = cj[j].batch;
-    }
-    switch (__builtin_amdgcn_readfirstlane(threadIdx.x / kRowsPerBlock)) {
-    case 0: quad_rows<KIND, GROUP, 0, XF, true>(J, geom, T, P, blk); break;
-    case 1: quad_rows<KIND, GROUP, 1, XF, true>(J, geom, T, P, blk); break;
-    case 2: quad_rows<KIND, GROUP, 2, XF, true>(J, geom, T, P, blk); break;
-    default: quad_rows<KIND, GROUP, 3, XF, true>(J, geom, T, P, blk); break;
-    }
-}
-
-// Activation pre-pass of the quarter GEMV: rot[v][0..dev) = per-group FWHT
+// Activation pre-pass of the quarter and batch GEMVs: rot[v][0..dev) = per-group FWHT
 // of zero-padded x (the reference's transform, cq.cpp:153-156, identical
 // butterflies), for nvec = count * batch vectors at once: vector v is row
 // v % batch of x0 (xptr null) or of xptr[v / batch] (a device table).
@@ -1307,41 +1177,19 @@ template <int GROUP>
 __global__ __launch_bounds__(kRowsPerBlock) void rot_many_kernel(const float *__restrict__ x0,
                                                                  const float *const *__restrict__ xptr, int batch,
                                                                  int in, int dev, float scale, float *__restrict__ rot) {
-    static_assert(GROUP <= 64, "in-wave FWHT");
+    static_assert(GROUP <= kWindow && kPositionsPerThread == 1, "one window per workgroup");
+    __shared__ float stage[GROUP > 64 ? kWindow : 1];
     const int v = blockIdx.y;
     const int p = blockIdx.x * kRowsPerBlock + threadIdx.x;
     const float *xv = (xptr ? xptr[v / batch] : x0) + static_cast<size_t>(v % batch) * in;
     float x[1] = {p < in ? xv[p] : 0.0f};
-    window_fwht<GROUP>(x, scale, nullptr);
+    window_fwht<GROUP>(x, scale, stage);
     if (p < dev) rot[static_cast<size_t>(v) * dev + p] = x[0];
 }
 
-// Batches of two or more rows on the 4-bit quarter GEMV take the pair kernel
-// (NEEDLE2_GPU_FP32_PAIRS=never: one row per pass). 2-bit matrices keep one
-// row per pass: their GEMV is bound by the table lookups, which pairs do not
-// reduce, and the pair kernel's one workgroup per CU runs them slower
-// (16 x 8192^2 at batch 2: 132 -> 183 us).
-static bool pairs_wanted(int max_batch) {
-    const char *mode = std::getenv("NEEDLE2_GPU_FP32_PAIRS");
-    return max_batch >= 2 && !(mode && std::strcmp(mode, "never") == 0);
-}
-
 template <int KIND, bool XF>
-void launch_gemv_kind(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, hipStream_t s,
-                      int max_batch) {
+void launch_gemv_kind(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, hipStream_t s) {
     dim3 grid(blocks), block(kRowsPerBlock), split(kSplitThreads), quad(kQuadThreads);
-    if constexpr (KIND == kNib) {  // (2-bit: LDS-bound, one row per pass)
-        if (g.group <= 64 && pairs_wanted(max_batch)) {
-            switch (g.group) {
-            case 8: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 8, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
-            case 16: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 16, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
-            case 32: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 32, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
-            default: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 64, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
-            }
-            ND_HIP(hipGetLastError());
-            return;
-        }
-    }
     switch (g.group > kWindow ? 0 : g.group) {
     case 8: hipLaunchKernelGGL((cq_gemv_quad_kernel<KIND, 8, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
     case 16: hipLaunchKernelGGL((cq_gemv_quad_kernel<KIND, 16, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
@@ -1493,7 +1341,9 @@ void launch_rot_many(const float *x0, const float *const *xptr, int batch, int n
     case 16: hipLaunchKernelGGL(rot_many_kernel<16>, grid, block, 0, s, x0, xptr, batch, in, dev, scale, rot); break;
     case 32: hipLaunchKernelGGL(rot_many_kernel<32>, grid, block, 0, s, x0, xptr, batch, in, dev, scale, rot); break;
     case 64: hipLaunchKernelGGL(rot_many_kernel<64>, grid, block, 0, s, x0, xptr, batch, in, dev, scale, rot); break;
-    default: throw Error("internal: activation pre-pass takes groups of 8 .. 64");
+    case 128: hipLaunchKernelGGL(rot_many_kernel<128>, grid, block, 0, s, x0, xptr, batch, in, dev, scale, rot); break;
+    case 256: hipLaunchKernelGGL(rot_many_kernel<256>, grid, block, 0, s, x0, xptr, batch, in, dev, scale, rot); break;
+    default: throw Error("internal: activation pre-pass takes groups of 8 .. 256");
     }
     ND_HIP(hipGetLastError());
 }
@@ -1503,7 +1353,7 @@ void launch_rot_many(const float *x0, const float *const *xptr, int batch, int n
 // pays where saving the pre-pass launch outweighs that: inputs of at most two
 // windows (the 8192 x 512 device call: 10.2 -> 6.7 us). NEEDLE2_GPU_FP32_XF =
 // always / never overrides.
-bool gemv_quad_takes_x(int group, int in) {
+static bool gemv_quad_takes_x(int group, int in) {
     if (group > 64) return false;
     const char *mode = std::getenv("NEEDLE2_GPU_FP32_XF");
     if (mode && std::strcmp(mode, "never") == 0) return false;
@@ -1511,17 +1361,29 @@ bool gemv_quad_takes_x(int group, int in) {
     return in <= 2 * kWindow;
 }
 
-void launch_cq_gemv(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, hipStream_t s,
-                    bool x_raw, int max_batch) {
+// Batches run the batch kernel (NEEDLE2_GPU_FP32_PAIRS=never: one row per
+// pass over the codes). Its buffer resource spans eight rows, which must stay
+// under 2^32 bytes.
+GemvPath gemv_path(int group, int in, int dev, int batch) {
+    const char *mode = std::getenv("NEEDLE2_GPU_FP32_PAIRS");
+    const bool batched = batch >= 2 && dev <= 1 << 26 && !(mode && std::strcmp(mode, "never") == 0);
+    return {batched, gemv_quad_takes_x(group, in) || (gemv_fuses_fwht(group) && !batched)};
+}
+
+void launch_cq_gemv(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, int batch,
+                    const GemvPath &path, hipStream_t s) {
     if (blocks <= 0) return;
-    ND_CHECK(!x_raw || g.group <= 64, "internal: raw GEMV input for a group the pre-pass does not serve");
-    if (x_raw) {
-        if (g.kind == kNib) launch_gemv_kind<kNib, true>(g, job0, jobs, njobs, blocks, s, max_batch);
-        else launch_gemv_kind<kCrumb, true>(g, job0, jobs, njobs, blocks, s, max_batch);
+    if (path.batched) {
+        launch_cq_gemv_batch(g, job0, jobs, njobs, blocks, batch, path.raw, s);
         return;
     }
-    if (g.kind == kNib) launch_gemv_kind<kNib, false>(g, job0, jobs, njobs, blocks, s, max_batch);
-    else launch_gemv_kind<kCrumb, false>(g, job0, jobs, njobs, blocks, s, max_batch);
+    if (path.raw && g.group <= 64) {
+        if (g.kind == kNib) launch_gemv_kind<kNib, true>(g, job0, jobs, njobs, blocks, s);
+        else launch_gemv_kind<kCrumb, true>(g, job0, jobs, njobs, blocks, s);
+        return;
+    }
+    if (g.kind == kNib) launch_gemv_kind<kNib, false>(g, job0, jobs, njobs, blocks, s);
+    else launch_gemv_kind<kCrumb, false>(g, job0, jobs, njobs, blocks, s);
 }
 
 void launch_gather_rows(const uint4 *codes, const uint16_t *norms, int rows, int chunks, int groups,

@@ -68,10 +68,9 @@ struct Mat {
 };
 
 // Row tiles of several CQ matrices that share one input, run as one GEMV
-// launch (matrices of one geometry) after at most one activation transform.
-// The job table holds `tokens` copies of the pieces, token-major, each over
-// its token's input row and into its token's output rows, so a launch over
-// the first n tokens runs n times the workgroups of one token.
+// launch (matrices of one geometry) after at most one activation transform:
+// one job per piece, of one row for a single token (decode step) and of T
+// rows for a prompt chunk of T tokens. Both are bit-identical per token.
 struct GemvGroup {
     struct Piece {
         const Matrix *m;
@@ -80,12 +79,12 @@ struct GemvGroup {
         int ystride;      // floats between consecutive tokens' outputs
     };
     const Matrix *m0 = nullptr;
-    DevBuf<uint8_t> jobs;
+    DevBuf<uint8_t> jobs;  // `pieces` jobs of a single token, then those of a chunk
     DevBuf<float> rot, big;
-    int pieces = 0, per_token = 0;  // jobs and workgroups of one token
+    int pieces = 0, blocks = 0;  // jobs and row tiles of one launch
     const float *x = nullptr;
     CqJob job0{};
-    bool xraw = false;  // groups <= 64: the GEMV transforms the raw input itself
+    GemvPath one{}, many{};  // a single token's launch, a chunk's
 
     static bool compatible(const Matrix &a, const Matrix &b) {
         return a.in == b.in && a.bits == b.bits && a.group == b.group &&
@@ -96,46 +95,43 @@ struct GemvGroup {
     void build(const std::vector<Piece> &ps, const float *input, int tokens) {
         m0 = ps[0].m;
         x = input;
-        xraw = gemv_prepass(m0->group) && gemv_quad_takes_x(m0->group, m0->in);
-        const bool fused = gemv_fuses_fwht(m0->group) || xraw;
-        if (!fused) rot.reserve(size_t(m0->dev) * tokens);
+        one = gemv_path(m0->group, m0->in, m0->dev, 1);
+        many = gemv_path(m0->group, m0->in, m0->dev, tokens);
+        many.batched = true;  // the pieces' outputs are strided, which the one-row kernels do not write
+        many.raw = many.raw && m0->group <= 64;
+        if (!one.raw || !many.raw) rot.reserve(size_t(m0->dev) * tokens);
         std::vector<CqJob> host;
-        int blocks = 0;
-        for (int t = 0; t < tokens; ++t)
+        for (const GemvPath &path : {one, many}) {
+            blocks = 0;
             for (const Piece &p : ps) {
                 ND_CHECK(compatible(*m0, *p.m), "internal: GEMV group of mixed geometry");
                 const int tile0 = p.first / kRowsPerBlock;
                 const int tile1 = (p.first + p.rows - 1) / kRowsPerBlock;
                 const int tiles = tile1 - tile0 + 1;
                 const int rows = std::min(tiles * kRowsPerBlock, p.m->out - tile0 * kRowsPerBlock);
-                const float *act = fused ? input + size_t(t) * m0->in : rot.p + size_t(t) * m0->dev;
                 host.push_back(CqJob{p.m->codes.p + size_t(tile0) * p.m->chunks * kRowsPerBlock,
-                                     p.m->norms.p + size_t(tile0) * p.m->groups * kRowsPerBlock, act,
-                                     p.y + size_t(t) * p.ystride, rows, tiles * kRowsPerBlock, blocks, 1});
+                                     p.m->norms.p + size_t(tile0) * p.m->groups * kRowsPerBlock,
+                                     path.raw ? input : rot.p, p.y, rows, tiles * kRowsPerBlock, blocks, 1, p.ystride});
                 blocks += tiles;
             }
-        pieces = static_cast<int>(ps.size());
-        per_token = blocks / tokens;
-        job0 = host[0];
-        if (host.size() > 1) {
-            jobs.reserve(host.size() * sizeof(CqJob));
-            ND_HIP(hipMemcpy(jobs.p, host.data(), host.size() * sizeof(CqJob), hipMemcpyHostToDevice));
         }
+        pieces = static_cast<int>(ps.size());
+        job0 = host[0];
+        jobs.reserve(host.size() * sizeof(CqJob));
+        ND_HIP(hipMemcpy(jobs.p, host.data(), host.size() * sizeof(CqJob), hipMemcpyHostToDevice));
     }
 
     void run(hipStream_t s, int tokens) {
-        if (!gemv_fuses_fwht(m0->group) && !xraw) {
+        const GemvPath &path = tokens > 1 ? many : one;
+        if (!path.raw) {
             if (gemv_prepass(m0->group))
                 launch_rot_many(x, nullptr, tokens, tokens, m0->in, m0->dev, m0->group, m0->scale, rot.p, s);
             else
                 m0->transform(x, m0->in, rot.p, tokens, big, s);
         }
-        const int njobs = pieces * tokens;
-        if (njobs > 1)
-            launch_cq_gemv(m0->geom(), CqJob{}, reinterpret_cast<const CqJob *>(jobs.p), njobs, per_token * tokens, s,
-                           xraw);
-        else
-            launch_cq_gemv(m0->geom(), job0, nullptr, 0, per_token, s, xraw);
+        const auto *table = reinterpret_cast<const CqJob *>(jobs.p) + (tokens > 1 ? pieces : 0);
+        const bool by_value = tokens == 1 && pieces == 1;
+        launch_cq_gemv(m0->geom(), job0, by_value ? nullptr : table, by_value ? 0 : pieces, blocks, tokens, path, s);
     }
 };
 

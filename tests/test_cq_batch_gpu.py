@@ -1,0 +1,63 @@
+"""The FP32 batch GEMV (cq_batch.h): several activation rows per pass over the codes, products on the matrix cores.
+
+Bit-identical to the oracle at every tile height (2, 3, 4, 6, 8 rows, a last tile of fewer), for groups below, equal
+to and above one block of 64 positions, with the K walk in one part and in four (rows of at least four groups and
+256 positions), odd widths and rows, raw (up to 512 wide) and transformed inputs.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from openneedle_amd.cq import CQMatrix, Plan
+from openneedle_amd.device import DeviceArray, synchronize
+from tests.cases import activations, example
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("group", [8, 32, 64, 128, 512])
+@pytest.mark.parametrize("rows,dim,batch", [
+    (257, 1100, 2), (257, 1100, 3), (300, 2100, 7), (300, 513, 9),  # few tiles: four parts, low tiles
+    (64, 100, 6),                                                  # a row of few groups: one part
+    (1, 300, 2500), (520, 70, 1501),                               # many tiles: high ones, a short last one
+])
+def test_batch_tiles_and_parts(bits, group, rows, dim, batch):
+    packed, norms, cb, dense = example(bits, rows=rows, dim=dim, group=group, seed=group + rows + batch)
+    x = activations((batch, dim), seed=batch)
+    expected = oracle.cq_linear(packed, norms, dense.shape, bits, group, cb, x, 4)
+    q = CQMatrix(packed, norms, dense.shape, bits, group, cb)
+    np.testing.assert_array_equal(q.matvec(x), expected)
+
+
+def test_batch_plan_of_several_matrices():
+    """A plan's matrices of different row counts in one launch, each with its own input."""
+    made = [example(4, rows=r, dim=600, group=32, seed=r) for r in (33, 256, 700)]
+    xs = [activations((5, 600), seed=k) for k in range(3)]
+    d_x = [DeviceArray.from_host(x) for x in xs]
+    d_y = [DeviceArray(4 * 5 * m[3].shape[0]) for m in made]
+    mats = [CQMatrix(p, n, d.shape, 4, 32, cb) for p, n, cb, d in made]
+    plan = Plan(mats, [d.ptr for d in d_x], [d.ptr for d in d_y], batch=5)
+    plan.run()
+    synchronize()
+    for (p, n, cb, d), x, y in zip(made, xs, d_y):
+        expected = oracle.cq_linear(p, n, d.shape, 4, 32, cb, x, 4)
+        np.testing.assert_array_equal(y.download(np.empty(expected.shape, np.float32)), expected)
+
+
+def test_batch_special_values():
+    """Products that underflow to denormals or zero of either sign, infinities and NaN come out as the reference's
+    separately rounded products and sums do."""
+    packed, norms, cb, dense = example(4, rows=300, dim=512, group=64, seed=3)
+    x = activations((6, 512), seed=4)
+    x[0] *= 1e-38
+    x[1] *= 1e-44
+    x[2, ::2] = 0.0
+    x[2, 1::2] *= -1e-40
+    x[3] = -0.0
+    x[4, 7] = np.inf
+    x[5, 9] = np.nan
+    expected = oracle.cq_linear(packed, norms, dense.shape, 4, 64, cb, x, 4)
+    q = CQMatrix(packed, norms, dense.shape, 4, 64, cb)
+    got = q.matvec(x)
+    np.testing.assert_array_equal(got, expected)
