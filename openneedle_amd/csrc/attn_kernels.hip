@@ -25,6 +25,7 @@
 #include "wave.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace nd {
 
@@ -75,6 +76,72 @@ __global__ __launch_bounds__(256) void kv_store_kernel(KvStoreArgs a) {
 
 __device__ __forceinline__ float i8f(uint32_t w, int c) {
     return static_cast<float>(static_cast<int8_t>((w >> (8 * c)) & 0xffu));
+}
+
+// With a new token (no slot list, so list position = slot), wave 0 of the
+// block whose split holds slot new_slot[seq] (the last split for a slot past
+// every range; no block for one outside the cache) first stores the token's K
+// and V rows there as kv_store_kernel does; the block barrier (a
+// workgroup-scope release and acquire) orders those stores before the block's
+// loads of that slot, and no other block reads it. When the slot lies past the
+// waves' first sub-tiles, those loads are issued before the store.
+template <int HD>
+__device__ __forceinline__ void store_new(const AttnArgs &a, int ns, int seq, int kh, size_t row0) {
+    if (threadIdx.x < 64) {
+        const size_t src = (static_cast<size_t>(seq) * a.kvheads + kh) * HD;
+        const size_t dst = row0 + ns;
+        store_kv_row(a.new_k + src, a.new_v + src, HD, threadIdx.x, a.k8 + dst * HD, a.v8 + dst * HD, a.ks + dst,
+                     a.vs + dst);
+    }
+    __syncthreads();
+}
+
+// The block's result from its four waves' maxima, sums and outputs in LDS (NR
+// partial outputs per wave), each wave rescaled to the common maximum: the
+// output row (one split; also left prepared as the next projection's input),
+// or the split's record.
+template <int HD, int G, int NR>
+__device__ __forceinline__ void combine_waves(const AttnArgs &a, const float (&lm)[4][G], const float (&ll)[4][G],
+                                              const float (&lred)[4][NR][G][HD], int seq, int kh, int sp) {
+    const int t = threadIdx.x, lane = t & 63;
+    const int H = a.kvheads * G;
+    for (int i = t; i < G * HD; i += 256) {
+        const int g = i / HD, d = i % HD;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) M = fmaxf(M, lm[w][g]);
+        float o = 0.0f, lt = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (lm[w][g] == -INFINITY) continue;  // a wave with nothing attended
+            const float f = expf(lm[w][g] - M);
+            float ow = 0.0f;
+            for (int r = 0; r < NR; ++r) ow += lred[w][r][g][d];
+            o += f * ow;
+            lt += f * ll[w][g];
+        }
+        const size_t head = static_cast<size_t>(seq) * H + kh * G + g;
+        if (a.splits == 1) {
+            const float val = lt > 0 ? o * (1.0f / lt) : 0.0f;
+            a.out[head * HD + d] = val;
+            if (a.prep.q) {
+                // whole waves (G * HD is a multiple of 64) over consecutive positions of the sequence's
+                // output row: groups of 32 lanes are groups of the next projection's input
+                const PrepOut &po = a.prep;
+                const int p = (kh * G + g) * HD + d;
+                prepare_lane<32>(val, lane, p, po.padded, po.dev, po.scale, po.kind,
+                                 po.q + static_cast<size_t>(seq) * po.dev, po.xs + static_cast<size_t>(seq) * po.groups + p / 32,
+                                 po.xst + static_cast<size_t>(p / 32) * po.batch + seq);
+            }
+        } else {
+            float *rec = a.part + (head * a.splits + sp) * (HD + 2);
+            rec[2 + d] = o;
+            if (d == 0) {
+                rec[0] = M;
+                rec[1] = lt;
+            }
+        }
+    }
 }
 
 // Block (split, kv head, sequence): 4 waves, each an independent
@@ -216,23 +283,6 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
         asm volatile("" ::: "memory");
     };
 
-    // With a new token (no slot list, so list position = slot), wave 0 of
-    // the block whose split holds slot new_slot[seq] (the last split for a
-    // slot past every range; no block for one outside the cache) first stores
-    // the token's K and V rows there as kv_store_kernel does; the block
-    // barrier (a workgroup-scope release and acquire) orders those stores
-    // before the block's loads of that slot, and no other block reads it.
-    // When the slot lies past the waves' first sub-tiles, those loads are
-    // issued before the store.
-    auto store_new = [&](int ns) {
-        if (wave == 0) {
-            const size_t src = (static_cast<size_t>(seq) * a.kvheads + kh) * HD;
-            const size_t dst = row0 + ns;
-            store_kv_row(a.new_k + src, a.new_v + src, HD, lane, a.k8 + dst * HD, a.v8 + dst * HD, a.ks + dst,
-                         a.vs + dst);
-        }
-        __syncthreads();
-    };
     const int ns = a.new_k ? a.new_slot[seq] : -1;
     const bool store_here =
         a.new_k && ns >= 0 && static_cast<uint32_t>(ns) < cap && sp == min(ns / a.slots_per_split, a.splits - 1);
@@ -242,9 +292,9 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
     // end read zero.
     Tile cur, nxt;
     int st = begin + wave * 64;
-    if (store_early) store_new(ns);
+    if (store_early) store_new<HD>(a, ns, seq, kh, row0);
     load(cur, st);
-    if (store_here && !store_early) store_new(ns);
+    if (store_here && !store_early) store_new<HD>(a, ns, seq, kh, row0);
     for (; st < end; st += 256) {
         load(nxt, st + 256);
         asm volatile("" ::: "memory");  // keep the prefetch ahead of the compute
@@ -263,43 +313,330 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
         for (int c = 0; c < 4 * VW; ++c) lred[wave][vr][g][vj * 4 * VW + c] = acc[g][c];
     }
     __syncthreads();
-    for (int i = t; i < G * HD; i += 256) {
-        const int g = i / HD, d = i % HD;
-        float M = -INFINITY;
+    combine_waves<HD, G, NLW>(a, lm, ll, lred, seq, kh, sp);
+}
+
+// ---- several query heads per kv head: matrix cores on the int8 codes --------
+//
+// The vector kernel above does every (slot, head, d) term on the VALU, for G
+// heads G times (measured at 16 sequences x 8 kv heads x 4 heads x 4096 ragged
+// slots of 128: 64 us, 1.4 TB/s of cache). Here both products run on
+// v_mfma_i32_16x16x64_i8 (32 deep for rows of 32) straight from the int8
+// codes, so the cache stream bounds it.
+//
+// Scores. q is split once per block into four 7-bit digits of a 28-bit fixed
+// point number relative to its head's largest |q| (finer than fp32 there), and
+// the 16 rows of operand A are 4 heads x 4 digits. Operand B is 16 slots' K
+// codes. Output register v of lane l is digit v of head l / 16 and slot l % 16:
+// exact integer dots, joined in the lane with two integer shift-adds and one
+// fused multiply-add.
+//
+// Values. w = p * v_scale is split the same way relative to the largest w of
+// the head's 64 slots, its bytes transposed so that operand A's rows are heads
+// x digits and its depth the 64 slots; operand B is the V codes, whose rows a
+// lane loads HD / 16 consecutive bytes at a time (lane l: d = HD / 16 *
+// (l % 16) ..) for 16 slots and transposes with byte permutes (depth byte
+// 4 u + t of lane group l / 16 is slot 16 t + 4 (l / 16) + u). Output register v
+// of lane l is digit v of head l / 16, output d = HD / 16 * (l % 16) + i.
+//
+// The splits keep 27 (q) and 26 (w) bits below the largest term, so the result
+// is at least as close to the exact value as fp32 products and sums.
+template <int HD>
+struct MfmaShape {
+    static constexpr int kVB = HD / 16;               // V bytes per lane and slot
+    static constexpr int kVD = (kVB + 3) / 4;         // dwords of them
+    static constexpr int kKH = HD == 128 ? 2 : 1;     // operand registers of 16 (32: 8) bytes per K row and lane
+    static constexpr int kKB = HD == 32 ? 8 : 16;     // bytes of each
+};
+
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+typedef int32_t i32x2 __attribute__((ext_vector_type(2)));
+
+template <int HD>
+__device__ __forceinline__ i32x4 mfma_rows(const i32x4 &a, const i32x4 &b, const i32x4 &c) {
+    if constexpr (HD == 32)
+        return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, i32x2{a.x, a.y}),
+                                                     __builtin_bit_cast(long, i32x2{b.x, b.y}), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+}
+
+// D0 2^21 + D1 2^14 + D2 2^7 + D3 of integer digit sums |D| < 2^21.
+__device__ __forceinline__ float join_digits(const i32x4 &d) {
+    const int hi = d.x * 128 + d.y, lo = d.z * 128 + d.w;
+    return __builtin_fmaf(static_cast<float>(hi), 16384.0f, static_cast<float>(lo));
+}
+
+// 4 x 4 byte transpose: out[i] = byte i of in[0], in[1], in[2], in[3].
+__device__ __forceinline__ void transpose4(const uint32_t (&in)[4], uint32_t (&out)[4]) {
+    const uint32_t a = __builtin_amdgcn_perm(in[1], in[0], 0x05010400u);  // bytes 0, 0, 1, 1 of in[0], in[1]
+    const uint32_t b = __builtin_amdgcn_perm(in[1], in[0], 0x07030602u);
+    const uint32_t c = __builtin_amdgcn_perm(in[3], in[2], 0x05010400u);
+    const uint32_t d = __builtin_amdgcn_perm(in[3], in[2], 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+}
+
+// The largest of v over the 16 lanes l % 16 (floats, or absolute bit patterns).
+__device__ __forceinline__ uint32_t row_max(uint32_t v, int lane) {
+    auto step = [&](auto h) {
+        const uint32_t o =
+            __builtin_bit_cast(uint32_t, butterfly_partner<decltype(h)::value>(__builtin_bit_cast(float, v), lane));
+        v = v > o ? v : o;
+    };
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 4>{});
+    step(std::integral_constant<int, 8>{});
+    return v;
+}
+
+constexpr uint32_t kInfBits = 0x7F800000u;
+constexpr int kDigitBias = 64 * (1 + (1 << 7) + (1 << 14) + (1 << 21));
+
+// Block and waves as attn_kernel; sub-tiles of 64 slots as four groups t of 16.
+// Loads of slots not attended read zero (offsets past the buffer).
+template <int HD, int G, bool SLOTS>
+__global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
+    using S = MfmaShape<HD>;
+    constexpr int VB = S::kVB, VD = S::kVD, KH = S::kKH, KB = S::kKB;
+    constexpr int HQ = (G + 3) / 4;        // quads of heads
+    constexpr int GQ = G < 4 ? G : 4;      // heads of a quad
+    constexpr uint32_t kOut = 0x80000000u;  // past every buffer (capacity * HD < 2^31)
+    // A operand rows of the value product, 16 bytes of row m = 4 head + digit per 16 slots; a head's four rows
+    // are 80 words apart (the writes of the four heads fall in different banks)
+    __shared__ __attribute__((aligned(16))) uint32_t wd[4][HQ][4 * 80];
+    __shared__ float lred[4][1][G][HD];
+    __shared__ float lm[4][G], ll[4][G];
+
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int col = lane & 15, quad = lane >> 4;  // score lane: slot 16 t + col of head 4 hq + quad
+    const int sp = blockIdx.x, kh = blockIdx.y, seq = blockIdx.z;
+    const int H = a.kvheads * G;
+    int len = a.lengths ? a.lengths[seq] : a.length;
+    len = len < a.length ? len : a.length;
+    const int begin = sp * a.slots_per_split;
+    const int end = min(begin + a.slots_per_split, len);
+    const uint32_t cap = static_cast<uint32_t>(a.capacity);
+
+    const float *qh = a.q + (static_cast<size_t>(seq) * H + kh * G) * HD;
+    const size_t row0 = (static_cast<size_t>(a.shared_cache ? 0 : seq) * a.kvheads + kh) * cap;
+    const auto rk = buffer_rsrc(a.k8 + row0 * HD, cap * HD);
+    const auto rv = buffer_rsrc(a.v8 + row0 * HD, cap * HD);
+    const auto rks = buffer_rsrc(a.ks + row0, cap * 4u);
+    const auto rvs = buffer_rsrc(a.vs + row0, cap * 4u);
+    const auto rsl = buffer_rsrc(a.slots + static_cast<size_t>(seq) * a.slots_stride, static_cast<uint32_t>(a.length) * 4u);
+
+    // slot of list position s, or -1 when not attended
+    auto slot_of = [&](int s) -> int {
+        int raw = s;
+        if constexpr (SLOTS) raw = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rsl, s * 4u, 0, 0));
+        return (s < end && static_cast<uint32_t>(raw) < cap) ? raw : -1;
+    };
+
+    struct Tile {
+        i32x4 k[4][KH];
+        uint32_t v[4][4][VD];  // [u][t]
+        float ks[4], vs[4];
+        bool valid[4];
+    };
+    auto load = [&](Tile &T, int st) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) M = fmaxf(M, lm[w][g]);
-        float o = 0.0f, lt = 0.0f;
+        for (int i = 0; i < 4; ++i) {
+            const int slot = slot_of(st + 16 * i + col);
+            T.valid[i] = slot >= 0;
+            const uint32_t kb = slot >= 0 ? static_cast<uint32_t>(slot) * HD + quad * (KB * KH) : kOut;
+            const uint32_t sb = slot >= 0 ? static_cast<uint32_t>(slot) * 4u : kOut;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            if (lm[w][g] == -INFINITY) continue;  // a wave with nothing attended
-            const float f = expf(lm[w][g] - M);
-            float ow = 0.0f;
-            for (int r = 0; r < NLW; ++r) ow += lred[w][r][g][d];
-            o += f * ow;
-            lt += f * ll[w][g];
+            for (int h = 0; h < KH; ++h) {
+                if constexpr (KB == 16) {
+                    T.k[i][h] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, kb, h * 16, 0));
+                } else {
+                    const auto w = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(rk, kb, 0, 0));
+                    T.k[i][h] = i32x4{w.x, w.y, 0, 0};
+                }
+            }
+            T.ks[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rks, sb, 0, 0));
+            T.vs[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rvs, sb, 0, 0));
         }
-        const size_t head = static_cast<size_t>(seq) * H + kh * G + g;
-        if (a.splits == 1) {
-            const float val = lt > 0 ? o * (1.0f / lt) : 0.0f;
-            a.out[head * HD + d] = val;
-            if (a.prep.q) {
-                // whole waves (G * HD is a multiple of 64) over consecutive positions of the sequence's
-                // output row: groups of 32 lanes are groups of the next projection's input
-                const PrepOut &po = a.prep;
-                const int p = (kh * G + g) * HD + d;
-                prepare_lane<32>(val, lane, p, po.padded, po.dev, po.scale, po.kind,
-                                 po.q + static_cast<size_t>(seq) * po.dev, po.xs + static_cast<size_t>(seq) * po.groups + p / 32,
-                                 po.xst + static_cast<size_t>(p / 32) * po.batch + seq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int slot = slot_of(st + 16 * i + 4 * quad + u);
+                const uint32_t vb = slot >= 0 ? static_cast<uint32_t>(slot) * HD + col * VB : kOut;
+                if constexpr (VB == 8) {
+                    const auto w = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, vb, 0, 0));
+                    T.v[u][i][0] = w.x;
+                    T.v[u][i][VD - 1] = w.y;
+                } else if constexpr (VB == 4) {
+                    T.v[u][i][0] = __builtin_amdgcn_raw_buffer_load_b32(rv, vb, 0, 0);
+                } else {
+                    T.v[u][i][0] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rv, vb, 0, 0));
+                }
             }
-        } else {
-            float *rec = a.part + (head * a.splits + sp) * (HD + 2);
-            rec[2 + d] = o;
-            if (d == 0) {
-                rec[0] = M;
-                rec[1] = lt;
+    };
+
+    float m[HQ], l[HQ], acc[HQ][VB];
+#pragma unroll
+    for (int hq = 0; hq < HQ; ++hq) {
+        m[hq] = -INFINITY;
+        l[hq] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < VB; ++i) acc[hq][i] = 0.0f;
+    }
+
+    const int ns = a.new_k ? a.new_slot[seq] : -1;
+    const bool store_here =
+        a.new_k && ns >= 0 && static_cast<uint32_t>(ns) < cap && sp == min(ns / a.slots_per_split, a.splits - 1);
+    const bool store_early = store_here && ns < begin + 256;  // the slot may be in a first sub-tile
+    Tile cur, nxt;
+    int st = begin + wave * 64;
+    if (store_early) store_new<HD>(a, ns, seq, kh, row0);
+    load(cur, st);
+    if (store_here && !store_early) store_new<HD>(a, ns, seq, kh, row0);
+
+    // q as operand A: lane (row 4 g + digit, 16-byte chunk quad); qscale: of score lane's head
+    i32x4 q8[HQ][KH];
+    float qscale[HQ];
+#pragma unroll
+    for (int hq = 0; hq < HQ; ++hq) {
+        const int g = col >> 2, digit = col & 3;
+        const bool live = g < GQ;
+        const float *src = qh + (hq * 4 + (live ? g : 0)) * HD + quad * (KB * KH);
+        float x[KH][KB];
+        uint32_t top = 0;
+#pragma unroll
+        for (int h = 0; h < KH; ++h)
+#pragma unroll
+            for (int e = 0; e < KB; ++e) {
+                x[h][e] = live ? src[h * KB + e] : 0.0f;
+                const uint32_t bits = __builtin_bit_cast(uint32_t, x[h][e]) & 0x7FFFFFFFu;
+                top = top > bits ? top : bits;
             }
+        // over the row's four lanes
+        const uint32_t o16 = __builtin_bit_cast(uint32_t, butterfly_partner<16>(__builtin_bit_cast(float, top), lane));
+        top = top > o16 ? top : o16;
+        const uint32_t o32 = __builtin_bit_cast(uint32_t, butterfly_partner<32>(__builtin_bit_cast(float, top), lane));
+        top = top > o32 ? top : o32;
+        const int fe = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, top));  // |q| < 2^fe
+#pragma unroll
+        for (int h = 0; h < KH; ++h) {
+            uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < KB; ++e) {
+                // bias: 64 in every digit, so that the digits are unsigned and every byte (digit - 64) signed
+                const int y = __float2int_rn(ldexpf(x[h][e], 27 - fe)) + kDigitBias;
+                const int dg = digit == 0 ? y >> 21 : (y >> (7 * (3 - digit))) & 127;
+                w[e >> 2] |= (static_cast<uint32_t>(dg - 64) & 0xFFu) << (8 * (e & 3));
+            }
+            q8[hq][h] = i32x4{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
+        }
+        // an infinity or NaN in q makes the head's scores NaN, as its products would
+        const float sc = top >= kInfBits ? __builtin_nanf("") : ldexpf(1.0f, fe - 27);
+        qscale[hq] = __shfl(sc, 4 * quad);
+    }
+
+    auto compute = [&](const Tile &T) {
+        // V codes as operand B: depth byte 4 u + t
+        i32x4 vt[VB];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int w = 0; w < VD; ++w) {
+                const uint32_t in[4] = {T.v[u][0][w], T.v[u][1][w], T.v[u][2][w], T.v[u][3][w]};
+                uint32_t out[4];
+                transpose4(in, out);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (4 * w + i < VB) vt[4 * w + i][u] = static_cast<int>(out[i]);
+            }
+#pragma unroll
+        for (int hq = 0; hq < HQ; ++hq) {
+            float x[4];
+            float top = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                i32x4 d = {0, 0, 0, 0};
+#pragma unroll
+                for (int h = 0; h < KH; ++h) d = mfma_rows<HD>(q8[hq][h], T.k[i][h], d);
+                x[i] = join_digits(d) * qscale[hq] * T.ks[i];
+                x[i] *= a.scale;
+                x[i] = T.valid[i] ? x[i] : -INFINITY;
+                top = fmaxf(top, x[i]);
+            }
+            const float mn = fmaxf(m[hq], group_max<16>(top, lane));
+            const float alpha = mn == -INFINITY ? 1.0f : expf(m[hq] - mn);
+            m[hq] = mn;
+            float w[4];
+            uint32_t wtop = 0;
+            float ls = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float e = T.valid[i] ? expf(x[i] - mn) : 0.0f;
+                ls += e;
+                w[i] = e * T.vs[i];
+                const uint32_t bits = __builtin_bit_cast(uint32_t, w[i]) & 0x7FFFFFFFu;
+                wtop = wtop > bits ? wtop : bits;
+            }
+            l[hq] = l[hq] * alpha + ls;
+            wtop = row_max(wtop, lane);
+            const int fe = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, wtop));  // |w| < 2^fe
+            uint32_t y[4], z[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // 27 bits, biased by 64 in every digit; then 64 off every byte (|f| < 2^26: bytes stay below 128)
+                const uint32_t f = static_cast<uint32_t>(__float2int_rn(ldexpf(w[i], 26 - fe)) + kDigitBias);
+                y[i] = (f >> 21) | (f >> 6 & 0x7F00u) | (f << 9 & 0x7F0000u) | (f << 24 & 0x7F000000u);
+                y[i] = ((y[i] | 0x80808080u) - 0x40404040u) ^ 0x80808080u;
+            }
+            transpose4(y, z);  // z[digit]: bytes t = 0 .. 3
+            uint32_t *dst = wd[wave][hq] + quad * 80 + col;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[i * 16] = z[i];
+            // LDS operations of one wave complete in order; the fences only stop the compiler from moving the read
+            // above the writes (and the next writes above the read)
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
+            const i32x4 w8 = *reinterpret_cast<const i32x4 *>(wd[wave][hq] + (col >> 2) * 80 + (col & 3) * 16 + quad * 4);
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
+            // an infinite or NaN weight makes the head's outputs NaN
+            const float ws = wtop >= kInfBits ? __builtin_nanf("") : ldexpf(1.0f, fe - 26);
+#pragma unroll
+            for (int i = 0; i < VB; ++i) {
+                const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(w8, vt[i], i32x4{0, 0, 0, 0}, 0, 0, 0);
+                acc[hq][i] = __builtin_fmaf(join_digits(d), ws, acc[hq][i] * alpha);
+            }
+        }
+    };
+
+    for (; st < end; st += 256) {
+        load(nxt, st + 256);
+        asm volatile("" ::: "memory");  // keep the prefetch ahead of the compute
+        compute(cur);
+        cur = nxt;
+    }
+#pragma unroll
+    for (int hq = 0; hq < HQ; ++hq) {
+        float ws = l[hq];
+        ws += butterfly_partner<1>(ws, lane);
+        ws += butterfly_partner<2>(ws, lane);
+        ws += butterfly_partner<4>(ws, lane);
+        ws += butterfly_partner<8>(ws, lane);
+        if (quad < GQ) {
+            if (col == 0) {
+                lm[wave][hq * 4 + quad] = m[hq];
+                ll[wave][hq * 4 + quad] = ws;
+            }
+#pragma unroll
+            for (int i = 0; i < VB; ++i) lred[wave][0][hq * 4 + quad][col * VB + i] = acc[hq][i];
         }
     }
+    __syncthreads();
+    combine_waves<HD, G, 1>(a, lm, ll, lred, seq, kh, sp);
 }
 
 // One block per query head: out = sum_i exp(m_i - M) o_i / sum_i exp(m_i - M) l_i, in split order.
@@ -348,15 +685,15 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(const float *__restrict
     }
 }
 
-// 16-byte value loads (VW = 4) while the accumulators fit; single words for
-// 4 or 8 query heads per kv head.
+// One query head per kv head: the vector kernel (the matrix kernel leaves three
+// quarters of its score lanes idle there). Two and more: the matrix kernel.
 template <int HD, bool SLOTS>
 void launch_attn_hd(const AttnArgs &a, int G, dim3 grid, hipStream_t s) {
     switch (G) {
     case 1: hipLaunchKernelGGL((attn_kernel<HD, 1, 4, SLOTS>), grid, dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((attn_kernel<HD, 2, 4, SLOTS>), grid, dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((attn_kernel<HD, 4, 1, SLOTS>), grid, dim3(256), 0, s, a); break;
-    case 8: hipLaunchKernelGGL((attn_kernel<HD, 8, 1, SLOTS>), grid, dim3(256), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((attn_mfma_kernel<HD, 2, SLOTS>), grid, dim3(256), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((attn_mfma_kernel<HD, 4, SLOTS>), grid, dim3(256), 0, s, a); break;
+    case 8: hipLaunchKernelGGL((attn_mfma_kernel<HD, 8, SLOTS>), grid, dim3(256), 0, s, a); break;
     default: ND_CHECK(false, "attention: heads per kv head must be 1, 2, 4 or 8");
     }
     ND_HIP(hipGetLastError());
