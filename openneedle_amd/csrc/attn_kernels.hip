@@ -157,8 +157,9 @@ __device__ __forceinline__ void combine_waves(const AttnArgs &a, const float (&l
 // not attended (past the range, or outside [0, capacity) in the caller's
 // list) gets an offset past the buffer and reads zero without a memory
 // request, so loads need no branches.
-template <int HD, int G, int VW, bool SLOTS>
+template <int HD, bool SLOTS>
 __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
+    constexpr int G = 1, VW = 4;   // one query head per kv head; 16-byte value loads
     constexpr int DW = HD / 4;
     constexpr int LPR = DW / VW;   // lanes per value row
     constexpr int NLW = 64 / LPR;  // slot lanes per wave
@@ -685,12 +686,17 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(const float *__restrict
     }
 }
 
-// One query head per kv head: the vector kernel (the matrix kernel leaves three
-// quarters of its score lanes idle there). Two and more: the matrix kernel.
+// One query head per kv head leaves three quarters of the matrix kernel's score
+// lanes idle: at rows of 64 the vector kernel is ahead (64 sequences x 8 kv heads
+// x 2048 slots 24.4 against 24.9 us, one sequence 7.7 against 8.3), at rows of
+// 128 the matrix kernel (8 x 8 x up to 8192 slots 24.4 against 28.0 us).
 template <int HD, bool SLOTS>
 void launch_attn_hd(const AttnArgs &a, int G, dim3 grid, hipStream_t s) {
     switch (G) {
-    case 1: hipLaunchKernelGGL((attn_kernel<HD, 1, 4, SLOTS>), grid, dim3(256), 0, s, a); break;
+    case 1:
+        if constexpr (HD < 128) hipLaunchKernelGGL((attn_kernel<HD, SLOTS>), grid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((attn_mfma_kernel<HD, 1, SLOTS>), grid, dim3(256), 0, s, a);
+        break;
     case 2: hipLaunchKernelGGL((attn_mfma_kernel<HD, 2, SLOTS>), grid, dim3(256), 0, s, a); break;
     case 4: hipLaunchKernelGGL((attn_mfma_kernel<HD, 4, SLOTS>), grid, dim3(256), 0, s, a); break;
     case 8: hipLaunchKernelGGL((attn_mfma_kernel<HD, 8, SLOTS>), grid, dim3(256), 0, s, a); break;

@@ -2,7 +2,7 @@
 // on fp16 MFMA with fp32 accumulation (the batched form of cq.cpp:157-197,
 // as Engine::linear_batch uses it for prompt chunks, engine.cpp:607-670).
 //
-// 1. prefill_transform_wave_kernel (groups <= 64: FWHT in registers and lane
+// 1. prefill_transform_wave_kernel (groups <= 256: FWHT in registers and lane
 //    butterflies) / prefill_transform_kernel (larger groups: FWHT in LDS):
 //    per-group FWHT of X (the reference's stage order, then * 1/sqrt(group))
 //    written as fp16 in MFMA fragment order:
@@ -92,55 +92,81 @@ __global__ __launch_bounds__(256) void prefill_transform_kernel(const float *__r
     }
 }
 
-// Groups of 8 .. 64: one workgroup per (32-row block, 64-position step),
-// thread (row r, unit u) = lane 8 (r % 8) + u owns positions 64 s + 8 u .. + 8
-// of row r. FWHT stages 1, 2, 4 run on the thread's eight values, stages 8,
-// 16, 32 are lane butterflies at strides 1, 2, 4 (the reference's stage order
-// and operands, as transform_kernel); the thread writes its 16-byte slice of
-// the fragment layout (eight rows of a wave: 128 contiguous bytes per slice).
+// Groups of 8 .. 256: one workgroup per (32-row block, S = max(1, GROUP / 64)
+// steps of 64 positions), thread (row r, unit u) = lane 8 (r % 8) + u owns
+// positions 64 s + 8 u .. + 8 of row r in each of the steps. FWHT stages 1, 2,
+// 4 run on the thread's eight values, stages 8, 16, 32 are lane butterflies at
+// strides 1, 2, 4 and stages 64, 128 pair the thread's steps (the reference's
+// stage order and operands, as transform_kernel); the thread writes its
+// 16-byte slices of the fragment layout (eight rows of a wave: 128 contiguous
+// bytes per slice).
 template <int GROUP>
 __global__ __launch_bounds__(256) void prefill_transform_wave_kernel(const float *__restrict__ x, int m, int in,
                                                                      int padded, int dev, float scale,
                                                                      _Float16 *__restrict__ xf) {
-    static_assert(GROUP >= 8 && GROUP <= 64, "in-wave FWHT");
-    const int s = blockIdx.x, rb = blockIdx.y;
+    static_assert(GROUP >= 8 && GROUP <= 256, "in-register FWHT");
+    constexpr int S = GROUP > 64 ? GROUP / 64 : 1;
+    const int s0 = blockIdx.x * S, rb = blockIdx.y;
     const int t = threadIdx.x, u = t & 7, r = t >> 3;  // r: row in the block (0..31)
-    const int v = rb * 32 + r, p0 = s * kBK + 8 * u;
-    float a[8];
-    if (v < m && p0 + 8 <= in) {
-        const float4 *src = reinterpret_cast<const float4 *>(x + static_cast<size_t>(v) * in + p0);
-        if ((reinterpret_cast<uintptr_t>(src) & 15) == 0) {
-            const float4 lo = src[0], hi = src[1];
-            a[0] = lo.x, a[1] = lo.y, a[2] = lo.z, a[3] = lo.w, a[4] = hi.x, a[5] = hi.y, a[6] = hi.z, a[7] = hi.w;
+    const int v = rb * 32 + r;
+    float a[S][8];
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+        const int p0 = (s0 + i) * kBK + 8 * u;
+        if (v < m && p0 + 8 <= in) {
+            const float4 *src = reinterpret_cast<const float4 *>(x + static_cast<size_t>(v) * in + p0);
+            if ((reinterpret_cast<uintptr_t>(src) & 15) == 0) {
+                const float4 lo = src[0], hi = src[1];
+                a[i][0] = lo.x, a[i][1] = lo.y, a[i][2] = lo.z, a[i][3] = lo.w;
+                a[i][4] = hi.x, a[i][5] = hi.y, a[i][6] = hi.z, a[i][7] = hi.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a[i][e] = x[static_cast<size_t>(v) * in + p0 + e];
+            }
         } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) a[e] = x[static_cast<size_t>(v) * in + p0 + e];
+            for (int e = 0; e < 8; ++e) a[i][e] = v < m && p0 + e < in ? x[static_cast<size_t>(v) * in + p0 + e] : 0.0f;
         }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a[e] = v < m && p0 + e < in ? x[static_cast<size_t>(v) * in + p0 + e] : 0.0f;
     }
 #pragma unroll
-    for (int h = 1; h < 8; h <<= 1)
+    for (int i = 0; i < S; ++i) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (!(e & h)) {
-                const float lo = a[e], hi = a[e + h];
-                a[e] = lo + hi;
-                a[e + h] = lo - hi;
-            }
+        for (int h = 1; h < 8; h <<= 1)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) wave_butterflies<GROUP / 8, 1>(a[e], t);
-    uint32_t w[4];
+            for (int e = 0; e < 8; ++e)
+                if (!(e & h)) {
+                    const float lo = a[i][e], hi = a[i][e + h];
+                    a[i][e] = lo + hi;
+                    a[i][e + h] = lo - hi;
+                }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const _Float16 h0 = static_cast<_Float16>(p0 + 2 * q < padded ? a[2 * q] * scale : 0.0f);
-        const _Float16 h1 = static_cast<_Float16>(p0 + 2 * q + 1 < padded ? a[2 * q + 1] * scale : 0.0f);
-        w[q] = uint32_t(__builtin_bit_cast(uint16_t, h0)) | (uint32_t(__builtin_bit_cast(uint16_t, h1)) << 16);
+        for (int e = 0; e < 8; ++e) wave_butterflies<(GROUP < 64 ? GROUP : 64) / 8, 1>(a[i][e], t);
     }
+#pragma unroll
+    for (int h = 1; h < S; h <<= 1)
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            if (!(i & h))
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float lo = a[i][e], hi = a[i + h][e];
+                    a[i][e] = lo + hi;
+                    a[i + h][e] = lo - hi;
+                }
     const int kk = u & 3, hh = u >> 2;
-    const size_t idx = (((static_cast<size_t>(rb) * (dev / kBK) + s) * 4 + kk) * 64 + hh * 32 + r) * 8;
-    *reinterpret_cast<u32x4 *>(xf + idx) = u32x4{w[0], w[1], w[2], w[3]};
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+        const int p0 = (s0 + i) * kBK + 8 * u;
+        uint32_t w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const _Float16 h0 = static_cast<_Float16>(p0 + 2 * q < padded ? a[i][2 * q] * scale : 0.0f);
+            const _Float16 h1 = static_cast<_Float16>(p0 + 2 * q + 1 < padded ? a[i][2 * q + 1] * scale : 0.0f);
+            w[q] = uint32_t(__builtin_bit_cast(uint16_t, h0)) | (uint32_t(__builtin_bit_cast(uint16_t, h1)) << 16);
+        }
+        const size_t idx = (((static_cast<size_t>(rb) * (dev / kBK) + s0 + i) * 4 + kk) * 64 + hh * 32 + r) * 8;
+        *reinterpret_cast<u32x4 *>(xf + idx) = u32x4{w[0], w[1], w[2], w[3]};
+    }
 }
 
 // Code-pair table in LDS: entry e (a byte of codes: low nibble first) holds
@@ -162,8 +188,8 @@ struct GemmArgs {
 // each XCD a contiguous run of tiles (M-tile fastest) keeps the M-tiles of an
 // N-tile, which read the same codes, on one XCD's L2.
 __device__ __forceinline__ int gemm_tile(const GemmArgs &g) {
-    const int b = blockIdx.x;
-    return g.tiles % 8 ? b : (b & 7) * (g.tiles >> 3) + (b >> 3);
+    const int b = blockIdx.x, x = b & 7;
+    return x * (g.tiles >> 3) + min(x, g.tiles & 7) + (b >> 3);
 }
 
 // ---- MFMA waves ----------------------------------------------------------
@@ -246,6 +272,45 @@ __device__ __forceinline__ void mma_step(AFrags (&a)[3], BSlice (&b)[2], const G
     // step c + 1) while the reads of buffer (c + 1) % 3 (rewritten in step
     // c + 2) stay in flight. This wave writes no LDS.
     asm volatile("s_waitcnt lgkmcnt(4)\n\ts_barrier" ::: "memory");
+}
+
+// Tall tiles (256 rows): wave mi owns rows 64 mi .. + 64 and all 128 columns
+// over the whole of K, so a dequantized weight feeds twice the MFMAs. X
+// fragments: a ring of eight slices, each refilled two steps ahead as soon as
+// its MFMAs are issued (slices 4 (c % 2) + kk of the ring belong to step c).
+struct TallFrags {
+    u32x4 v[8][2];  // [slice of the ring][32-row block]
+};
+
+__device__ __forceinline__ void tall_load(TallFrags &a, int slot, int kk, const APtrs &p, int s) {
+    const int so = __builtin_amdgcn_readfirstlane(s * kStepBytes);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        a.v[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(p.x, p.xv[i] + kk * kFragBytes, so, 0);
+}
+
+template <int J>
+__device__ __forceinline__ void tall_step(TallFrags &a, BSlice (&b)[2], const GemmArgs &g, const APtrs &p, int c,
+                                          const _Float16 (&Bs)[3][kBN * kLdsRow], f16x (&acc)[2][4], int lane) {
+    const int ahead = min(c + 2, g.ksteps - 1);  // clamped: past the end it repeats the last step
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        const int slot = 4 * (J & 1) + kk;
+        // the next slice's weights (after the last, the first of step c + 1; past the end: never used)
+        if (kk < 3) b_slice(b[(kk + 1) & 1], Bs[J % 3], kk + 1, lane);
+        else b_slice(b[0], Bs[(J + 1) % 3], 0, lane);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a.v[slot][i]), b[kk & 1].v[j],
+                                                                   acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        tall_load(a, slot, kk, p, ahead);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(4)\n\ts_barrier" ::: "memory");  // as mma_step
 }
 
 // ---- dequantization waves ------------------------------------------------
@@ -384,8 +449,23 @@ __device__ __forceinline__ void store_block(const f16x (&acc)[2][4], const u32x4
     }
 }
 
-template <int NG>
+// Row block I of a tall tile's wave, stored to Y.
+template <int I>
+__device__ __forceinline__ void store_rows(const f16x (&acc)[2][4], const GemmArgs &g, int m_base, int n0, int lane) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int n = n0 + j * 32 + (lane & 31);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int m = m_base + I * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+            if (n < g.rows && m < g.m) g.y[static_cast<size_t>(m) * g.rows + n] = acc[I][j][e];
+        }
+    }
+}
+
+template <int NG, bool TALL>
 __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) {
+    constexpr int BM = TALL ? 2 * kBM : kBM;
     __shared__ __attribute__((aligned(16))) _Float16 Bs[3][kBN * kLdsRow];
     __shared__ __attribute__((aligned(16))) uint32_t pairs[kPairWords];
     // all 512 threads fill the code-pair table (16 x 16-byte stores each)
@@ -396,13 +476,42 @@ __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) 
     }
     __syncthreads();
     const int tile = gemm_tile(g);
-    const int n0 = (tile / g.mtiles) * kBN, m0 = (tile % g.mtiles) * kBM;
+    const int n0 = (tile / g.mtiles) * kBN, m0 = (tile % g.mtiles) * BM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int last = g.ksteps - 1;
     // Every step ends in one barrier on both sides; the loops run in sixes so
     // that every ring index is a compile-time constant.
-    if (wave < 4) {
+    if (TALL && wave < 4) {
+        const APtrs p = a_ptrs(g, m0 / 32 + 2 * wave, 0, lane);
+        f16x acc[2][4];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = f16x{};
+        TallFrags a;
+        BSlice b[2];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) tall_load(a, q, q & 3, p, min(q >> 2, last));
+        __syncthreads();  // weights of steps 0 and 1 are in LDS
+        b_slice(b[0], Bs[0], 0, lane);
+        int c = 0;
+        for (; c + 6 <= g.ksteps; c += 6) {
+            tall_step<0>(a, b, g, p, c, Bs, acc, lane);
+            tall_step<1>(a, b, g, p, c + 1, Bs, acc, lane);
+            tall_step<2>(a, b, g, p, c + 2, Bs, acc, lane);
+            tall_step<3>(a, b, g, p, c + 3, Bs, acc, lane);
+            tall_step<4>(a, b, g, p, c + 4, Bs, acc, lane);
+            tall_step<5>(a, b, g, p, c + 5, Bs, acc, lane);
+        }
+        if (c < g.ksteps) tall_step<0>(a, b, g, p, c, Bs, acc, lane);
+        if (c + 1 < g.ksteps) tall_step<1>(a, b, g, p, c + 1, Bs, acc, lane);
+        if (c + 2 < g.ksteps) tall_step<2>(a, b, g, p, c + 2, Bs, acc, lane);
+        if (c + 3 < g.ksteps) tall_step<3>(a, b, g, p, c + 3, Bs, acc, lane);
+        if (c + 4 < g.ksteps) tall_step<4>(a, b, g, p, c + 4, Bs, acc, lane);
+        store_rows<0>(acc, g, m0 + wave * 64, n0, lane);
+        store_rows<1>(acc, g, m0 + wave * 64, n0, lane);
+    } else if (wave < 4) {
         const int mi = wave >> 1, ki = wave & 1;
         const APtrs p = a_ptrs(g, m0 / 32 + 2 * mi, ki, lane);
         f16x acc[2][4];
@@ -470,7 +579,7 @@ __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) 
         if (c + 2 < g.ksteps) deq_step<NG, 2>(r, v, g, p, c + 2, pairs, lane4, Bs, row, ch);
         if (c + 3 < g.ksteps) deq_step<NG, 3>(r, v, g, p, c + 3, pairs, lane4, Bs, row, ch);
         if (c + 4 < g.ksteps) deq_step<NG, 4>(r, v, g, p, c + 4, pairs, lane4, Bs, row, ch);
-        __syncthreads();  // the MFMA waves' K-half exchange
+        if constexpr (!TALL) __syncthreads();  // the MFMA waves' K-half exchange
     }
 }
 
@@ -483,13 +592,15 @@ void launch_prefill_transform(const float *x, int m, int in, int padded, int dev
     if (m <= 0) return;
     ND_CHECK(group <= 16384, "prefill GEMM: group must be <= 16384");
     ND_CHECK(dev % kBK == 0, "internal: prefill rows must be whole 64-position steps");
-    if (group <= 64) {
-        dim3 grid(dev / kBK, (m + 31) / 32), block(256);
+    if (group <= kWindow) {  // dev is a whole number of windows
+        dim3 grid(dev / (group > kBK ? group : kBK), (m + 31) / 32), block(256);
         switch (group) {
         case 8: hipLaunchKernelGGL(prefill_transform_wave_kernel<8>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
         case 16: hipLaunchKernelGGL(prefill_transform_wave_kernel<16>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
         case 32: hipLaunchKernelGGL(prefill_transform_wave_kernel<32>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
-        default: hipLaunchKernelGGL(prefill_transform_wave_kernel<64>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
+        case 64: hipLaunchKernelGGL(prefill_transform_wave_kernel<64>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
+        case 128: hipLaunchKernelGGL(prefill_transform_wave_kernel<128>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
+        default: hipLaunchKernelGGL(prefill_transform_wave_kernel<256>, grid, block, 0, s, x, m, in, padded, dev, scale, xf); break;
         }
         ND_HIP(hipGetLastError());
         return;
@@ -500,6 +611,26 @@ void launch_prefill_transform(const float *x, int m, int in, int padded, int dev
                        scale, xf, seg);
     ND_HIP(hipGetLastError());
 }
+
+namespace {
+
+bool tall_tiles(int ntiles, int m) {
+    const int low = (ntiles * ((m + kBM - 1) / kBM) + 255) / 256;
+    const int tall = (ntiles * ((m + 2 * kBM - 1) / (2 * kBM)) + 255) / 256;
+    return tall * 1.4 < low;
+}
+
+template <bool TALL>
+void launch_gemm_tiles(const GemmArgs &g, dim3 grid, dim3 block, hipStream_t s) {
+    switch (g.group_shift) {
+    case 3: hipLaunchKernelGGL((prefill_gemm_kernel<4, TALL>), grid, block, 0, s, g); break;
+    case 4: hipLaunchKernelGGL((prefill_gemm_kernel<2, TALL>), grid, block, 0, s, g); break;
+    default: hipLaunchKernelGGL((prefill_gemm_kernel<1, TALL>), grid, block, 0, s, g); break;
+    }
+    ND_HIP(hipGetLastError());
+}
+
+}  // namespace
 
 void launch_prefill_gemm(const CqGeom &geom, const uint4 *codes4, int chunks4, const uint16_t *norms, int rows,
                          const _Float16 *xf, int m, int dev, int padded, const uint16_t *cb_half, float *y,
@@ -520,16 +651,15 @@ void launch_prefill_gemm(const CqGeom &geom, const uint4 *codes4, int chunks4, c
     g.group_shift = __builtin_ctz(static_cast<unsigned>(geom.group));
     g.xsteps = dev / kBK;
     g.ksteps = (padded + kBK - 1) / kBK;  // dev is a multiple of 256: whole steps stay in the row
-    g.mtiles = (m + kBM - 1) / kBM;
-    g.tiles = (rows + kBN - 1) / kBN * g.mtiles;
+    const int ntiles = (rows + kBN - 1) / kBN;
+    const bool tall = tall_tiles(ntiles, m);
+    const int bm = tall ? 2 * kBM : kBM;
+    g.mtiles = (m + bm - 1) / bm;
+    g.tiles = ntiles * g.mtiles;
     for (int i = 0; i < 16; ++i) g.cb[i] = cb_half[i];
     dim3 grid(g.tiles), block(kGemmThreads);
-    switch (g.group_shift) {
-    case 3: hipLaunchKernelGGL(prefill_gemm_kernel<4>, grid, block, 0, s, g); break;
-    case 4: hipLaunchKernelGGL(prefill_gemm_kernel<2>, grid, block, 0, s, g); break;
-    default: hipLaunchKernelGGL(prefill_gemm_kernel<1>, grid, block, 0, s, g); break;
-    }
-    ND_HIP(hipGetLastError());
+    if (tall) launch_gemm_tiles<true>(g, grid, block, s);
+    else launch_gemm_tiles<false>(g, grid, block, s);
 }
 
 namespace {
