@@ -296,6 +296,10 @@ void launch_sdot_quantize(const float *rot, int rot_stride, int nvec, int padded
 // The batch (uniform across jobs) is processed in tiles that decode each code once.
 void launch_sdot_gemv(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs_dev, int njobs, int total_blocks,
                       int batch, hipStream_t s);
+// sdot_batch.hip: 4-bit codes, batches of 2 and more, groups of 32 .. 1024; false, with nothing launched, for other shapes and rows
+// whose scales exceed its LDS.
+bool launch_sdot_batch(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs_dev, int njobs, int total_blocks,
+                       int batch, hipStream_t s);
 // As launch_sdot_gemv for the K-split kernel's shapes (small matrices, batch
 // 2 and more, groups 32 .. 256), with 32-row workgroups whose outputs of each
 // batch row, one group of 32 positions of the next projection's input, are

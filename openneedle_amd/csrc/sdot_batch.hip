@@ -1,0 +1,358 @@
+// gfx950 int8 ("SDOT") GEMV of 4-bit codes for batches of 2 .. 16 activation
+// rows and groups of 32 and more:
+//   value[b][row] += (float(dot_g) * (half(norm) * cs)) * x_scale[b][g]
+// for g in group order (sdot.cpp:43-44, 142-149), bit-identical to the
+// kernels of sdot_kernels.hip.
+//
+// What bounds those at a few rows is the VALU: 1.6 instructions a code to turn
+// codes into int8 centroids, and four instructions per (weight row, batch row,
+// group), for whole quads or sixteens of batch rows. Here
+// - codes and activations are multiplied as fp16: integers up to 127 are exact
+//   there, their products and sums of up to 1024 of them exact in the fp32
+//   accumulators, so the matrix cores deliver float(dot) itself and the
+//   epilogue is three instructions for the batch rows there are;
+// - a byte of codes is looked up as a pair of fp16 centroids, in a 256-entry
+//   LDS table with a column per lane (one v_perm and one conflict-free 4-byte
+//   read): half a VALU instruction a code;
+// - v_mfma_f32_4x4x4_16b_f16 takes 4 batch rows x 4 positions x 64 weight rows:
+//   lane l feeds its own weight row's codes (B) and ends up with its sums, and
+//   one register pair holds 4 batch rows x 64 positions of activations (A),
+//   block abid broadcast to all by cbsz = 4, so activations are loaded once per
+//   64 positions straight from memory and converted there.
+#include "common.h"
+#include "wave.h"
+
+#include <hip/hip_fp16.h>
+
+#include <type_traits>
+#include <utility>
+
+namespace nd {
+
+namespace {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+
+constexpr int kSdBlock = 64;                  // positions handled between two rounds of loads
+constexpr int kSdPairTable = 256 * 64;        // dwords of the 4-bit pair table
+constexpr int kSdAhead = 4;                   // code dwords looked up ahead of their products
+constexpr size_t kSdMaxLds = 160 * 1024;
+
+template <int GROUP, int NB>
+struct SdShape {
+    static constexpr int kQuads = (NB + 3) / 4;
+    static constexpr int kDwords = kSdBlock / 8;  // code dwords per block
+    static constexpr int kChunks = kDwords / 4;
+    static constexpr int kNorms = GROUP < kSdBlock ? kSdBlock / GROUP : 1;  // groups closing in a block
+    static constexpr int kScaleRow = kQuads * 4;                            // floats per group in LDS
+};
+
+template <int GROUP, int NB>
+struct SdState {
+    using S = SdShape<GROUP, NB>;
+    u32x4 codes[S::kChunks];
+    u32x2v q[S::kQuads];
+    uint16_t norms[S::kNorms];
+};
+
+// The lane's four activations (batch row l % 4, positions 4 (l / 4) .. + 4 of
+// the block) as fp16, from the prepared int8 codes of 8 positions, even ones
+// first. A byte b ^ 0x80 under 0x64 is the fp16 number 1024 + 128 + value.
+__device__ __forceinline__ h4 sd_halves(const u32x2v &q, uint32_t sel) {
+    const uint32_t t = __builtin_amdgcn_perm(q.y, q.x, sel) ^ 0x80808080u;
+    const h2v bias = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
+    const h2v lo = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, t, 0x04010400u)) + bias;
+    const h2v hi = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, t, 0x04030402u)) + bias;
+    return h4{lo.x, lo.y, hi.x, hi.y};
+}
+
+// fp16 centroid pairs of one code dword, positions in order: byte offset
+// 256 * (code byte k) + 4 * lane.
+__device__ __forceinline__ void sd_pairs(uint32_t (&v)[4], const uint32_t *table, uint32_t dword, uint32_t lane4) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        v[k] = *reinterpret_cast<const uint32_t *>(
+            reinterpret_cast<const char *>(table) +
+            __builtin_amdgcn_perm(dword, lane4, 0x0c0c0400u + (static_cast<uint32_t>(k) << 8)));
+}
+
+template <class F, int... I>
+__device__ __forceinline__ void sd_for_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void sd_for(F &&f) {
+    sd_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// KS parts of 256 threads share a row tile: part k takes rounds k, KS + k, ...
+// of max(64, GROUP) positions, parts above 0 park their group terms and part 0
+// adds them in group order, one round behind.
+template <int GROUP, int NB, int KS>
+struct SdPark {
+    static constexpr int kFloats = KS > 1 ? (KS - 1) * SdShape<GROUP, NB>::kNorms * NB * kRowsPerBlock : 0;
+    static constexpr int kTotal = 2 * kFloats;  // two rounds
+};
+
+template <int GROUP, int NB, int KS, bool FIRST>
+__device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, const uint32_t *table, float *park,
+                                        const float *scales, int blk, int b0, int part) {
+    using S = SdShape<GROUP, NB>;
+    constexpr int NN = S::kNorms, NQ = S::kQuads, D = S::kDwords;
+    constexpr int PF = SdPark<GROUP, NB, KS>::kFloats;
+    const int r = threadIdx.x % kRowsPerBlock, lane = threadIdx.x & 63;
+    const int tile = blk - J.block_begin;
+    const int nb = min(NB, J.batch - b0);
+    const int dev = geom.windows * kWindow;  // activation bytes per batch row
+    const __amdgpu_buffer_rsrc_t codes =
+        buffer_rsrc(J.codes + static_cast<size_t>(tile) * geom.chunks * kRowsPerBlock,
+                    static_cast<uint32_t>(geom.chunks) * kRowsPerBlock * 16u);
+    const __amdgpu_buffer_rsrc_t norms = buffer_rsrc(J.norms + static_cast<size_t>(tile) * geom.groups * kRowsPerBlock,
+                                                     static_cast<uint32_t>(geom.groups) * kRowsPerBlock * 2u);
+    const __amdgpu_buffer_rsrc_t acts =
+        buffer_rsrc(reinterpret_cast<const int8_t *>(J.q) + static_cast<size_t>(b0) * dev, static_cast<uint32_t>(nb) * dev);
+    const uint32_t code_lane = r * 16u, norm_lane = r * 2u, lane4 = lane * 4u;
+    const int bpg_shift = GROUP < kSdBlock ? 0 : __builtin_ctz(geom.group / kSdBlock);
+    const int i4 = lane >> 2;  // the lane's positions 4 i4 .. of the block
+    uint32_t xv[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)  // rows past the batch repeat its last row; their outputs are not stored
+        xv[q] = static_cast<uint32_t>(min(4 * q + (lane & 3), nb - 1)) * dev + (i4 >> 1) * 8;
+    // bytes of the lane's positions in the loaded dwords
+    const uint32_t sel = (i4 & 1) ? 0x07030602u : 0x05010400u;
+    const int groups = geom.groups;
+    const int bpg = 1 << bpg_shift;
+    const int blocks = GROUP < kSdBlock ? (groups + NN - 1) / NN : groups << bpg_shift;
+    const int rounds = (blocks + (KS << bpg_shift) - 1) / (KS << bpg_shift);
+    const int count = rounds << bpg_shift;
+    auto block_of = [&](int n) { return (((n >> bpg_shift) * KS + part) << bpg_shift) + (n & (bpg - 1)); };
+    auto load_chunk = [&](int block, int c) {
+        return __builtin_amdgcn_raw_buffer_load_b128(
+            codes, code_lane, __builtin_amdgcn_readfirstlane((block * S::kChunks + c) * kRowsPerBlock * 16), kStreamLoad);
+    };
+    auto load_rest = [&](SdState<GROUP, NB> &s, int block) {
+        const int so = __builtin_amdgcn_readfirstlane(block * kSdBlock);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            s.q[q] = __builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(acts, xv[q], so, 0));
+#pragma unroll
+        for (int k = 0; k < NN; ++k) {  // a group past the last reads zero and is never added
+            const int g = GROUP < kSdBlock ? block * NN + k : block >> bpg_shift;
+            s.norms[k] = __builtin_amdgcn_raw_buffer_load_b16(
+                norms, norm_lane, __builtin_amdgcn_readfirstlane(g * kRowsPerBlock * 2), 0);
+        }
+    };
+    SdState<GROUP, NB> st[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+#pragma unroll
+        for (int c = 0; c < S::kChunks; ++c) st[n].codes[c] = load_chunk(block_of(n), c);
+        load_rest(st[n], block_of(n));
+    }
+    float value[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) value[b] = 0.0f;
+    f4 acc[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t w[D][4];  // centroid pairs of the block's code dwords, kSdAhead of them in flight
+    static_assert(kSdAhead == 4 && D == 8, "the dwords read ahead are one chunk");
+    const u32x4 c0 = st[0].codes[0];
+    sd_pairs(w[0], table, c0.x, lane4);
+    sd_pairs(w[1], table, c0.y, lane4);
+    sd_pairs(w[2], table, c0.z, lane4);
+    sd_pairs(w[3], table, c0.w, lane4);
+
+    auto add_parked = [&](int it) {
+        const float *src = park + (it & 1) * PF + r;
+#pragma unroll
+        for (int k = 1; k < KS; ++k)
+#pragma unroll
+            for (int j = 0; j < NN; ++j)
+                if ((it * KS + k) * NN + j < groups)
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) value[b] += src[(((k - 1) * NN + j) * NB + b) * kRowsPerBlock];
+    };
+    // k: which of the block's groups; xs: its activation scales
+    auto close = [&](int it, int k, uint16_t norm, const float (&xs)[NQ * 4]) {
+        const float ns = __half2float(__ushort_as_half(norm)) * geom.centroid_scale;  // sdot.cpp:43-44
+        if constexpr (FIRST) {
+            if (it * KS * NN + k < groups)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) value[b] = value[b] + (acc[b / 4][b & 3] * ns) * xs[b];
+        } else {
+            float *dst = park + (it & 1) * PF + r;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) dst[(((part - 1) * NN + k) * NB + b) * kRowsPerBlock] = (acc[b / 4][b & 3] * ns) * xs[b];
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) acc[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    // One block: centroid pairs are read four code dwords ahead (a dword is about
+    // 60 clocks of work at 8 rows, an LDS read about 130), spent registers are
+    // refilled two blocks ahead.
+    auto block_step = [&](auto slot, int n) {
+        constexpr int cur = decltype(slot)::value;
+        SdState<GROUP, NB> &s = st[cur], &t = st[cur ^ 1];
+        const int it = n >> bpg_shift;
+        const int ahead = block_of(n + 2), here = block_of(n);
+        if constexpr (FIRST && KS > 1) {
+            if ((n & (bpg - 1)) == 0 && it > 0) add_parked(it - 1);
+        }
+        float xs[NN][NQ * 4];
+#pragma unroll
+        for (int k = 0; k < NN; ++k) {
+            const int g = min(GROUP < kSdBlock ? here * NN + k : here >> bpg_shift, groups - 1);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const float4 v = *reinterpret_cast<const float4 *>(scales + g * S::kScaleRow + 4 * q);
+                xs[k][4 * q] = v.x;
+                xs[k][4 * q + 1] = v.y;
+                xs[k][4 * q + 2] = v.z;
+                xs[k][4 * q + 3] = v.w;
+            }
+        }
+        h4 a[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) a[q] = sd_halves(s.q[q], sel);
+        sd_for<D>([&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            constexpr int dn = d + kSdAhead, e = dn & 3;
+            const u32x4 &cn = dn < D ? s.codes[dn / 4 % S::kChunks] : t.codes[0];
+            sd_pairs(w[dn % D], table, e == 0 ? cn.x : e == 1 ? cn.y : e == 2 ? cn.z : cn.w, lane4);
+            if constexpr (d == 0) s.codes[0] = load_chunk(ahead, 0);       // read during the previous block
+            if constexpr (dn == D - 1) s.codes[1] = load_chunk(ahead, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            sd_for<2>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                constexpr int P = 2 * d + i;  // four positions 4 P .. + 4
+                const h4 b = __builtin_bit_cast(h4, u32x2v{w[d][2 * i], w[d][2 * i + 1]});
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) acc[q] = __builtin_amdgcn_mfma_f32_4x4x4f16(a[q], b, acc[q], 4, P, 0);
+                if constexpr (GROUP < kSdBlock && 4 * (P + 1) % GROUP == 0)
+                    close(it, 4 * (P + 1) / GROUP - 1, s.norms[4 * (P + 1) / GROUP - 1], xs[4 * (P + 1) / GROUP - 1]);
+            });
+            // pins the dword's products and sums before the next dword's reads
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) asm volatile("" : "+v"(acc[q]));
+#pragma unroll
+            for (int b = 0; b < NB; ++b) asm volatile("" : "+v"(value[b]));
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (GROUP >= kSdBlock) {
+            if ((n & (bpg - 1)) == bpg - 1) close(it, 0, s.norms[0], xs[0]);
+        }
+        load_rest(s, ahead);
+        if constexpr (KS > 1) {
+            if ((n & (bpg - 1)) == bpg - 1) __syncthreads();
+        }
+    };
+    int n = 0;
+    for (; n + 2 <= count; n += 2) {
+        block_step(std::integral_constant<int, 0>{}, n);
+        block_step(std::integral_constant<int, 1>{}, n + 1);
+    }
+    if (n < count) block_step(std::integral_constant<int, 0>{}, n);
+    if constexpr (FIRST) {
+        if constexpr (KS > 1) add_parked(rounds - 1);
+        const int row = tile * kRowsPerBlock + r;
+        const size_t ys = J.ystride ? J.ystride : J.rows;
+        if (row < J.rows) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                if (b < nb) ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0 + b) * ys + row] = value[b];
+        }
+    }
+}
+
+template <int GROUP, int NB, int KS>
+__global__ __launch_bounds__(kRowsPerBlock *KS, 2) void sdot_batch_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
+                                                                        int njobs, SdotGeom geom) {
+    using S = SdShape<GROUP, NB>;
+    extern __shared__ __attribute__((aligned(16))) uint32_t sd_lds[];
+    uint32_t *table = sd_lds;
+    float *park = reinterpret_cast<float *>(sd_lds + kSdPairTable);
+    float *scales = park + SdPark<GROUP, NB, KS>::kTotal;  // [groups][kScaleRow]
+    const int blk = blockIdx.x, b0 = blockIdx.y * NB;
+    SdotJob J = job0;
+    if (njobs > 0) {
+        const ND_CONST SdotJob *cj = (const ND_CONST SdotJob *)(jobs);
+        const int j = find_job(cj, njobs, blk);
+        J.codes = cj[j].codes;
+        J.norms = cj[j].norms;
+        J.q = cj[j].q;
+        J.xs = cj[j].xs;
+        J.y = cj[j].y;
+        J.rows = cj[j].rows;
+        J.block_begin = cj[j].block_begin;
+        J.batch = cj[j].batch;
+        J.ystride = cj[j].ystride;
+    }
+    auto half_of = [&](int code) {  // the code's int8 centroid as fp16
+        const int c = static_cast<int8_t>((geom.cent[code >> 2] >> (8 * (code & 3))) & 0xFFu);
+        return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(c))));
+    };
+    for (int i = threadIdx.x; i < kSdPairTable / 4; i += kRowsPerBlock * KS) {  // 16 stores of 4 columns per entry
+        const int e = i >> 4;
+        const uint32_t v = half_of(e & 15) | half_of(e >> 4) << 16;
+        reinterpret_cast<u32x4 *>(table)[i] = u32x4{v, v, v, v};
+    }
+    const int nb = min(NB, J.batch - b0);
+    for (int i = threadIdx.x; i < geom.groups * S::kScaleRow; i += kRowsPerBlock * KS) {
+        const int g = i / S::kScaleRow, b = i % S::kScaleRow;
+        scales[i] = b < nb ? J.xs[static_cast<size_t>(b0 + b) * geom.groups + g] : 0.0f;
+    }
+    __syncthreads();
+    const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kRowsPerBlock) : 0;
+    if (part == 0) sd_rows<GROUP, NB, KS, true>(J, geom, table, park, scales, blk, b0, 0);
+    else sd_rows<GROUP, NB, KS, KS == 1>(J, geom, table, park, scales, blk, b0, part);
+}
+
+template <int GROUP, int NB, int KS>
+bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
+                     hipStream_t s) {
+    using S = SdShape<GROUP, NB>;
+    const size_t lds = (static_cast<size_t>(kSdPairTable) + SdPark<GROUP, NB, KS>::kTotal +
+                        static_cast<size_t>(g.groups) * S::kScaleRow) * 4;
+    if (lds > kSdMaxLds) return false;
+    const dim3 grid(blocks, (batch + NB - 1) / NB), block(kRowsPerBlock * KS);
+    hipLaunchKernelGGL((sdot_batch_kernel<GROUP, NB, KS>), grid, block, lds, s, job0, jobs, njobs, g);
+    ND_HIP(hipGetLastError());
+    return true;
+}
+
+template <int GROUP>
+bool sd_launch_group(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
+                     hipStream_t s) {
+    const int tiles = (batch + 15) / 16, rows = (batch + tiles - 1) / tiles;  // batch rows of a tile, all alike
+    auto go = [&](auto nb) {
+        constexpr int NB = decltype(nb)::value;
+        // up to one workgroup per CU: two parts over K
+        if (NB <= 8 && static_cast<long>(blocks) * tiles <= 256 && g.groups >= 4)
+            return sd_launch_shape<GROUP, NB, NB <= 8 ? 2 : 1>(g, job0, jobs, njobs, blocks, batch, s);
+        return sd_launch_shape<GROUP, NB, 1>(g, job0, jobs, njobs, blocks, batch, s);
+    };
+    if (rows <= 2) return go(std::integral_constant<int, 2>{});
+    if (rows <= 3) return go(std::integral_constant<int, 3>{});
+    if (rows <= 4) return go(std::integral_constant<int, 4>{});
+    if (rows <= 5) return go(std::integral_constant<int, 5>{});
+    if (rows <= 6) return go(std::integral_constant<int, 6>{});
+    if (rows <= 8) return go(std::integral_constant<int, 8>{});
+    if (rows <= 12) return go(std::integral_constant<int, 12>{});
+    return go(std::integral_constant<int, 16>{});
+}
+
+}  // namespace
+
+bool launch_sdot_batch(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
+                       hipStream_t s) {
+    // sums of up to 1024 products of int8 values stay below 2^24; a tile's activations below 2^32 bytes
+    if (g.kind != kNib || g.group < 32 || g.group > 1024 || batch < 2 || g.windows > 1 << 19) return false;
+    if (g.group == 32) return sd_launch_group<32>(g, job0, jobs, njobs, blocks, batch, s);
+    return sd_launch_group<64>(g, job0, jobs, njobs, blocks, batch, s);  // 64 .. 1024
+}
+
+}  // namespace nd

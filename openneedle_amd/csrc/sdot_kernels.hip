@@ -810,6 +810,11 @@ void launch_sdot_row(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs
 // DOTS the int32 group dots themselves are stored (dots[b][row][g]).
 // ---------------------------------------------------------------------------
 constexpr int kQuadMaxLds = 160 * 1024;
+// LDS rows of activations carry padding dwords, so that the batch rows that one
+// read touches lie in different banks (unpadded, every row of a power-of-two
+// width starts in the same bank: the 16-row reads of tile16 serialised
+// 16-fold).
+constexpr int kRowPad = 4;
 
 template <int KIND, int GROUP, int NQ, bool DOTS>
 __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
@@ -837,10 +842,11 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, 
     const int groups = geom.groups;
     const int dev = geom.windows * kWindow;
     const int qdw = dev / 4;  // activation dwords per batch row
+    const int ldw = qdw + kRowPad;  // and in LDS
     const int b0 = static_cast<int>(blockIdx.y) * TB;
     const int nb = min(TB, J.batch - b0);  // valid batch rows of the tile (uniform)
     uint32_t *lq = quad_lds;
-    float *lxs = reinterpret_cast<float *>(quad_lds + TB * qdw);
+    float *lxs = reinterpret_cast<float *>(quad_lds + TB * ldw);
     const uint32_t cent[4] = {geom.cent[0], geom.cent[1], geom.cent[2], geom.cent[3]};
     const float cs = geom.centroid_scale;
     const __amdgpu_buffer_rsrc_t codes =
@@ -855,7 +861,8 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, 
     // stage the tile's activation rows and group scales (rows past the batch as zeros)
     const u32x4 *q4 = reinterpret_cast<const u32x4 *>(J.q) + static_cast<size_t>(b0) * (qdw / 4);
     for (int i = threadIdx.x; i < TB * qdw / 4; i += kRowsPerBlock)
-        reinterpret_cast<u32x4 *>(lq)[i] = i / (qdw / 4) < nb ? q4[i] : u32x4{0, 0, 0, 0};
+        reinterpret_cast<u32x4 *>(lq)[i + i / (qdw / 4) * (kRowPad / 4)] =
+            i / (qdw / 4) < nb ? q4[i] : u32x4{0, 0, 0, 0};
     for (int i = threadIdx.x; i < TB * groups; i += kRowsPerBlock)
         lxs[i] = i / groups < nb ? J.xs[static_cast<size_t>(b0) * groups + i] : 0.0f;
     __syncthreads();
@@ -881,7 +888,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, 
             }
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const uint32_t *qa = lq + (4 * q + lb) * qdw + c * QPC + d * W;
+                const uint32_t *qa = lq + (4 * q + lb) * ldw + c * QPC + d * W;
 #pragma unroll
                 for (int m = 0; m < W; ++m)
                     acc[q] = __builtin_amdgcn_mfma_i32_4x4x4i8(static_cast<int>(qa[m]), static_cast<int>(wq[m]), acc[q],
@@ -944,7 +951,7 @@ bool launch_sdot_quad(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
                       int32_t *dots, hipStream_t s) {
     const int dev = g.windows * kWindow;
     const int tb = batch >= 16 ? 16 : (batch + 3) / 4 * 4;  // rows per tile
-    const size_t lds = static_cast<size_t>(tb) * dev + static_cast<size_t>(tb) * g.groups * 4;
+    const size_t lds = static_cast<size_t>(tb) * (dev + 4 * kRowPad) + static_cast<size_t>(tb) * g.groups * 4;
     if (lds > kQuadMaxLds || g.group > kWindow) return false;
     dim3 grid(blocks, (batch + tb - 1) / tb), block(kRowsPerBlock);
     auto go = [&](auto nq) {
@@ -1027,10 +1034,11 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     const int groups = geom.groups;
     const int dev = geom.windows * kWindow;
     const int qdw = dev / 4;
+    const int ldw = qdw + kRowPad;  // dwords of a batch row in LDS
     const int b0 = static_cast<int>(blockIdx.y) * TB;
     const int nb = min(TB, J.batch - b0);
     uint32_t *lq = t16_lds;
-    float *lxs = reinterpret_cast<float *>(t16_lds + TB * qdw);
+    float *lxs = reinterpret_cast<float *>(t16_lds + TB * ldw);  // [groups][16]
     const uint32_t cent[4] = {geom.cent[0], geom.cent[1], geom.cent[2], geom.cent[3]};
     const float cs = geom.centroid_scale;
     const __amdgpu_buffer_rsrc_t codes =
@@ -1063,9 +1071,10 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     // stage the tile's activation rows and group scales (rows past the batch as zeros)
     const u32x4 *q4 = reinterpret_cast<const u32x4 *>(J.q) + static_cast<size_t>(b0) * (qdw / 4);
     for (int i = threadIdx.x; i < TB * qdw / 4; i += kRowsPerBlock)
-        reinterpret_cast<u32x4 *>(lq)[i] = i / (qdw / 4) < nb ? q4[i] : u32x4{0, 0, 0, 0};
+        reinterpret_cast<u32x4 *>(lq)[i + i / (qdw / 4) * (kRowPad / 4)] =
+            i / (qdw / 4) < nb ? q4[i] : u32x4{0, 0, 0, 0};
     for (int i = threadIdx.x; i < TB * groups; i += kRowsPerBlock)
-        lxs[i] = i / groups < nb ? J.xs[static_cast<size_t>(b0) * groups + i] : 0.0f;
+        lxs[i % groups * TB + i / groups] = i / groups < nb ? J.xs[static_cast<size_t>(b0) * groups + i] : 0.0f;
     __syncthreads();
     float value[4][4];  // [m][r]: weight row wrow + 16 m + jr, batch row 4 t + r
 #pragma unroll
@@ -1075,10 +1084,9 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     v4i acc[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) acc[m] = v4i{0, 0, 0, 0};
-    const uint32_t *qrow = lq + jr * qdw + 2 * H * t;  // batch row jr: the activation dwords of code dword t
-    const float *xrow = lxs + 4 * t * groups;      // scales of batch rows 4t .. 4t + 3
-    auto chunk = [&](const Tile16Slot &sl, int c, bool closes) {
-        long a[H];
+    const uint32_t *qrow = lq + jr * ldw + 2 * H * t;  // batch row jr: the activation dwords of code dword t
+    const float *xrow = lxs + 4 * t;               // scales of batch rows 4t .. 4t + 3
+    auto read_a = [&](long (&a)[H], int c) {
         if constexpr (KIND == kNib) {
             const auto q2 = *reinterpret_cast<const uint32_t __attribute__((ext_vector_type(2))) *>(qrow + c * 8);
             a[0] = static_cast<long>(q2[0]) | (static_cast<long>(q2[1]) << 32);
@@ -1087,6 +1095,13 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
             a[0] = static_cast<long>(q4v.x) | (static_cast<long>(q4v.y) << 32);
             a[1] = static_cast<long>(q4v.z) | (static_cast<long>(q4v.w) << 32);
         }
+    };
+    long ahead[2][H];
+    read_a(ahead[0], 0);
+    // kc: c modulo 2; the next chunk's activations are read before this one's products (past the end: the last's)
+    auto chunk = [&](const Tile16Slot &sl, int c, int kc, bool closes) {
+        const long (&a)[H] = ahead[kc];
+        read_a(ahead[kc ^ 1], min(c + 1, nch - 1));
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             uint32_t wq[2 * H];  // the centroid dwords of code dword t, in activation-dword order
@@ -1115,9 +1130,8 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
                             dots[(static_cast<size_t>(b0 + 4 * t + r) * J.rows + row) * groups + g] = acc[m][r];
                 }
             } else {
-                float xsb[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) xsb[r] = xrow[r * groups + g];
+                const float4 xs4 = *reinterpret_cast<const float4 *>(xrow + g * TB);
+                const float xsb[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
                     const float ns = h2f(sl.norm[m]) * cs;  // sdot.cpp:43-44
@@ -1134,13 +1148,13 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     for (; c0 + kRowRing <= nch; c0 += kRowRing) {
 #pragma unroll
         for (int k = 0; k < kRowRing; ++k) {
-            chunk(ring[k], c0 + k, (k + 1) % CPG == 0);
+            chunk(ring[k], c0 + k, k & 1, (k + 1) % CPG == 0);
             load(ring[k], min(c0 + k + kRowRing, nch - 1), (k + 1) % CPG == 0);
         }
     }
 #pragma unroll
     for (int k = 0; k < kRowRing; ++k)
-        if (c0 + k < nch) chunk(ring[k], c0 + k, (k + 1) % CPG == 0);
+        if (c0 + k < nch) chunk(ring[k], c0 + k, k & 1, (k + 1) % CPG == 0);
     if constexpr (!DOTS) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -1158,7 +1172,7 @@ template <int KIND, bool DOTS>
 bool launch_sdot_tile16(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                         int32_t *dots, hipStream_t s) {
     const int dev = g.windows * kWindow;
-    const size_t lds = static_cast<size_t>(16) * dev + static_cast<size_t>(16) * g.groups * 4;
+    const size_t lds = static_cast<size_t>(16) * (dev + 4 * kRowPad) + static_cast<size_t>(16) * g.groups * 4;
     if (g.group < (KIND == kNib ? 32 : 64) || g.group > kWindow || lds > kQuadMaxLds) return false;
     dim3 grid(blocks, (batch + 15) / 16), block(kRowsPerBlock);
     switch (g.group) {
@@ -1824,6 +1838,19 @@ static bool tile16_wanted(int batch) {
     return batch > 8;
 }
 
+// The fp16 batch kernel (sdot_batch.hip) from 2 rows up (NEEDLE2_GPU_INT8_BATCH
+// "always" / "never"; an override of one of the kernels it stands before
+// leaves it out).
+static bool batch_wanted() {
+    const char *mode = std::getenv("NEEDLE2_GPU_INT8_BATCH");
+    if (mode && (std::strcmp(mode, "always") == 0 || std::strcmp(mode, "never") == 0)) return mode[0] == 'a';
+    for (const char *name : {"NEEDLE2_GPU_INT8_TILE16", "NEEDLE2_GPU_INT8_QUAD", "NEEDLE2_GPU_INT8_MFMA"}) {
+        const char *other = std::getenv(name);
+        if (other && (std::strcmp(other, "always") == 0 || std::strcmp(other, "never") == 0)) return false;
+    }
+    return true;
+}
+
 // The K split for small matrices (NEEDLE2_GPU_INT8_KSPLIT "always" / "never") and, within it, the 16 x 16
 // tiles (batch 2 and more; NEEDLE2_GPU_INT8_KS16 "never", or "always" from batch 1).
 static bool ks_chosen(const SdotGeom &g, int blocks, int batch) {
@@ -1906,6 +1933,7 @@ void launch_sdot_gemv(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
         else launch_sdot_row<kCrumb, false>(g, job0, jobs, njobs, blocks, nullptr, s);
         return;
     }
+    if (batch >= 2 && batch_wanted() && launch_sdot_batch(g, job0, jobs, njobs, blocks, batch, s)) return;
     if (!mfma_forced && tile16_wanted(batch)) {
         const bool done = g.kind == kNib ? launch_sdot_tile16<kNib, false>(g, job0, jobs, njobs, blocks, batch, nullptr, s)
                                          : launch_sdot_tile16<kCrumb, false>(g, job0, jobs, njobs, blocks, batch, nullptr, s);
