@@ -149,6 +149,28 @@ hipStream_t Staging::stream() {
     if (!stream_) ND_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     return stream_;
 }
+// The stream writes the call's number to pinned memory behind its kernels and
+// the host spins on it, with a look at the stream (for an error) now and then:
+// a 2048 x 512 CQ4 host-pointer product takes 20.7 us against 23.2 with
+// hipStreamSynchronize and 29.7 polling hipStreamQuery alone.
+void Staging::wait_written() {
+    if (!done.p) {
+        done.reserve(1);
+        *done.p = calls;
+    }
+    const uint32_t call = ++calls;
+    if (hipStreamWriteValue32(stream(), done.p, call, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        ND_HIP(hipStreamSynchronize(stream()));
+        return;
+    }
+    for (unsigned spins = 1; __atomic_load_n(done.p, __ATOMIC_ACQUIRE) != call; ++spins) {
+        if (spins % (1 << 22)) continue;  // about every 2 ms: a query delays the call by some 8 us
+        const hipError_t q = hipStreamQuery(stream());
+        if (q == hipSuccess) return;
+        if (q != hipErrorNotReady) ND_HIP(q);
+    }
+}
 Staging::~Staging() {
     if (stream_) (void)hipStreamDestroy(stream_);
 }
@@ -286,7 +308,7 @@ void CqHandle::linear_host(const float *x, float *y, int batch) {
         dx = st.x.p;
     }
     run_device(dx, st.hy.p, batch, st.stream());
-    ND_HIP(hipStreamSynchronize(st.stream()));
+    st.wait_written();
     std::memcpy(y, st.hy.p, ny * sizeof(float));
 }
 
@@ -430,7 +452,7 @@ void SdotHandle::linear_host(const float *x, float *y, int batch) {
         dx = st.x.p;
     }
     run_device(dx, st.hy.p, batch, st.stream());
-    ND_HIP(hipStreamSynchronize(st.stream()));
+    st.wait_written();
     std::memcpy(y, st.hy.p, ny * sizeof(float));
 }
 

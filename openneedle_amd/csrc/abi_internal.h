@@ -73,6 +73,10 @@ struct Staging {
     DevBuf<int32_t> ids;
     DevBuf<float> yfull;    // all outputs, when most rows are candidates
     HostBuf<float> hx, hy;
+    HostBuf<uint32_t> done;  // wait_written's flag
+    uint32_t calls = 0;
+    // Waits for the work on stream() whose last kernel wrote pinned host memory.
+    void wait_written();
     HostBuf<int32_t> hids;
     DevBuf<uint8_t> jobs;   // per-call job tables (needle2_cq_linear_many)
     HostBuf<uint8_t> hjobs;
