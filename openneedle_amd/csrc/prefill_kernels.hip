@@ -468,13 +468,22 @@ __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) 
     constexpr int BM = TALL ? 2 * kBM : kBM;
     __shared__ __attribute__((aligned(16))) _Float16 Bs[3][kBN * kLdsRow];
     __shared__ __attribute__((aligned(16))) uint32_t pairs[kPairWords];
-    // all 512 threads fill the code-pair table (16 x 16-byte stores each)
-    for (int i = threadIdx.x; i < kPairWords / 4; i += kGemmThreads) {
-        const int e = i >> 4;  // 16 vectors of 4 lanes per entry
-        const uint32_t v = uint32_t(g.cb[e & 15]) | (uint32_t(g.cb[e >> 4]) << 16);
-        reinterpret_cast<u32x4 *>(pairs)[i] = u32x4{v, v, v, v};
-    }
-    __syncthreads();
+    // all 512 threads fill the code-pair table (16 x 16-byte stores each), behind their first loads
+    auto fill_pairs = [&] {
+        // 16 vectors of 4 lanes per entry: the thread's entries share the low code, and the high one is
+        // uniform (no indexed read of the arguments)
+        const int low = (threadIdx.x >> 4) & 15;
+        uint32_t lo = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) lo = low == i ? g.cb[i] : lo;
+        const bool odd = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0;
+#pragma unroll
+        for (int k = 0; k < kPairWords / 4 / kGemmThreads; ++k) {
+            const uint32_t v = lo | static_cast<uint32_t>(odd ? g.cb[2 * k + 1] : g.cb[2 * k]) << 16;
+            reinterpret_cast<u32x4 *>(pairs)[threadIdx.x + k * kGemmThreads] = u32x4{v, v, v, v};
+        }
+        __syncthreads();
+    };
     const int tile = gemm_tile(g);
     const int n0 = (tile / g.mtiles) * kBN, m0 = (tile % g.mtiles) * BM;
     const int lane = threadIdx.x & 63;
@@ -493,6 +502,7 @@ __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) 
         BSlice b[2];
 #pragma unroll
         for (int q = 0; q < 8; ++q) tall_load(a, q, q & 3, p, min(q >> 2, last));
+        fill_pairs();
         __syncthreads();  // weights of steps 0 and 1 are in LDS
         b_slice(b[0], Bs[0], 0, lane);
         int c = 0;
@@ -523,6 +533,7 @@ __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) 
         BSlice b[2];
         a_load(a[0], p, 0);
         a_load(a[1], p, min(1, last));
+        fill_pairs();
         __syncthreads();  // weights of steps 0 and 1 are in LDS
         b_slice(b[0], Bs[0], 2 * ki, lane);
         int c = 0;
@@ -559,6 +570,7 @@ __global__ __launch_bounds__(kGemmThreads) void prefill_gemm_kernel(GemmArgs g) 
         uint32_t v[16];
 #pragma unroll
         for (int k = 0; k < 5; ++k) code_load(r[k], g, p, min(k, last));
+        fill_pairs();
         table_reads(v, r[0], pairs, lane4);
         scale_store(v, r[0], Bs[0], row, ch);
         table_reads(v, r[1], pairs, lane4);
