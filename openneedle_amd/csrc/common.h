@@ -32,9 +32,10 @@ const char *get_error();
 // Waits for the stream by polling it instead of hipStreamSynchronize, whose
 // wake-up measured 2-10% of an engine decode step (~650 us of kernels that end
 // by writing pinned host memory); the host thread spins while the stream runs.
-// Calls that end with an asynchronous device-to-host copy measured slower with
-// it (a 2048 x 512 host-pointer GEMV: 23 -> 27-31 us) and keep
-// hipStreamSynchronize.
+// Short calls measured slower with it (a 2048 x 512 host-pointer GEMV: 23 ->
+// 27-31 us): those wait on a value written by the stream
+// (Staging::wait_written), or keep hipStreamSynchronize where they end with a
+// copy.
 inline void wait_stream(hipStream_t s) {
     for (hipError_t q = hipStreamQuery(s); q != hipSuccess; q = hipStreamQuery(s))
         if (q != hipErrorNotReady) ND_HIP(q);
@@ -171,9 +172,10 @@ __host__ __device__ inline size_t norm_index(int r, int g, int groups) {
 
 // Where the FP32 GEMV's activations are transformed. One row: groups of 128
 // and 256 inside the kernel, groups up to 64 in a pre-pass (launch_rot_many)
-// or inside the quarter-split kernel (gemv_quad_takes_x). Batches: groups up
-// to 64 as for one row, 128 and 256 in the pre-pass. Groups above one window
-// always use the generic transform pass.
+// or inside the quarter-split kernel (narrow inputs). Batches: groups up to 64
+// as for one row, 128 and 256 in the pre-pass (groups of 128 transformed by
+// the batch kernel itself measured slower: a 512-token engine prompt 4.87 ->
+// 5.24 ms). Groups above one window always use the generic transform pass.
 inline bool gemv_fuses_fwht(int group) { return group > 64 && group <= kWindow; }
 
 // Largest group the int8 path's one-launch prepare (FWHT + quantize in LDS) takes.

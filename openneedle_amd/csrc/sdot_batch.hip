@@ -1,5 +1,5 @@
-// gfx950 int8 ("SDOT") GEMV of 4-bit codes for batches of 2 .. 16 activation
-// rows and groups of 32 and more:
+// gfx950 int8 ("SDOT") GEMV of 4-bit codes for batches of activation rows
+// (tiles of up to 12) and groups of 32 and more:
 //   value[b][row] += (float(dot_g) * (half(norm) * cs)) * x_scale[b][g]
 // for g in group order (sdot.cpp:43-44, 142-149), bit-identical to the
 // kernels of sdot_kernels.hip.
@@ -88,21 +88,11 @@ __device__ __forceinline__ void sd_for(F &&f) {
     sd_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// KS parts of 256 threads share a row tile: part k takes rounds k, KS + k, ...
-// of max(64, GROUP) positions, parts above 0 park their group terms and part 0
-// adds them in group order, one round behind.
-template <int GROUP, int NB, int KS>
-struct SdPark {
-    static constexpr int kFloats = KS > 1 ? (KS - 1) * SdShape<GROUP, NB>::kNorms * NB * kRowsPerBlock : 0;
-    static constexpr int kTotal = 2 * kFloats;  // two rounds
-};
-
-template <int GROUP, int NB, int KS, bool FIRST>
-__device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, const uint32_t *table, float *park,
-                                        const float *scales, int blk, int b0, int part) {
+template <int GROUP, int NB>
+__device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, const uint32_t *table,
+                                        const float *scales, int blk, int b0) {
     using S = SdShape<GROUP, NB>;
     constexpr int NN = S::kNorms, NQ = S::kQuads, D = S::kDwords;
-    constexpr int PF = SdPark<GROUP, NB, KS>::kFloats;
     const int r = threadIdx.x % kRowsPerBlock, lane = threadIdx.x & 63;
     const int tile = blk - J.block_begin;
     const int nb = min(NB, J.batch - b0);
@@ -126,9 +116,6 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
     const int groups = geom.groups;
     const int bpg = 1 << bpg_shift;
     const int blocks = GROUP < kSdBlock ? (groups + NN - 1) / NN : groups << bpg_shift;
-    const int rounds = (blocks + (KS << bpg_shift) - 1) / (KS << bpg_shift);
-    const int count = rounds << bpg_shift;
-    auto block_of = [&](int n) { return (((n >> bpg_shift) * KS + part) << bpg_shift) + (n & (bpg - 1)); };
     auto load_chunk = [&](int block, int c) {
         return __builtin_amdgcn_raw_buffer_load_b128(
             codes, code_lane, __builtin_amdgcn_readfirstlane((block * S::kChunks + c) * kRowsPerBlock * 16), kStreamLoad);
@@ -149,8 +136,8 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
 #pragma unroll
-        for (int c = 0; c < S::kChunks; ++c) st[n].codes[c] = load_chunk(block_of(n), c);
-        load_rest(st[n], block_of(n));
+        for (int c = 0; c < S::kChunks; ++c) st[n].codes[c] = load_chunk(n, c);
+        load_rest(st[n], n);
     }
     float value[NB];
 #pragma unroll
@@ -166,28 +153,12 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
     sd_pairs(w[2], table, c0.z, lane4);
     sd_pairs(w[3], table, c0.w, lane4);
 
-    auto add_parked = [&](int it) {
-        const float *src = park + (it & 1) * PF + r;
-#pragma unroll
-        for (int k = 1; k < KS; ++k)
-#pragma unroll
-            for (int j = 0; j < NN; ++j)
-                if ((it * KS + k) * NN + j < groups)
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) value[b] += src[(((k - 1) * NN + j) * NB + b) * kRowsPerBlock];
-    };
-    // k: which of the block's groups; xs: its activation scales
-    auto close = [&](int it, int k, uint16_t norm, const float (&xs)[NQ * 4]) {
+    // closes group g: xs, its activation scales
+    auto close = [&](int g, uint16_t norm, const float (&xs)[NQ * 4]) {
         const float ns = __half2float(__ushort_as_half(norm)) * geom.centroid_scale;  // sdot.cpp:43-44
-        if constexpr (FIRST) {
-            if (it * KS * NN + k < groups)
+        if (g < groups)
 #pragma unroll
-                for (int b = 0; b < NB; ++b) value[b] = value[b] + (acc[b / 4][b & 3] * ns) * xs[b];
-        } else {
-            float *dst = park + (it & 1) * PF + r;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) dst[(((part - 1) * NN + k) * NB + b) * kRowsPerBlock] = (acc[b / 4][b & 3] * ns) * xs[b];
-        }
+            for (int b = 0; b < NB; ++b) value[b] = value[b] + (acc[b / 4][b & 3] * ns) * xs[b];
 #pragma unroll
         for (int q = 0; q < NQ; ++q) acc[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     };
@@ -197,15 +168,11 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
     auto block_step = [&](auto slot, int n) {
         constexpr int cur = decltype(slot)::value;
         SdState<GROUP, NB> &s = st[cur], &t = st[cur ^ 1];
-        const int it = n >> bpg_shift;
-        const int ahead = block_of(n + 2), here = block_of(n);
-        if constexpr (FIRST && KS > 1) {
-            if ((n & (bpg - 1)) == 0 && it > 0) add_parked(it - 1);
-        }
+        const int ahead = n + 2;
         float xs[NN][NQ * 4];
 #pragma unroll
         for (int k = 0; k < NN; ++k) {
-            const int g = min(GROUP < kSdBlock ? here * NN + k : here >> bpg_shift, groups - 1);
+            const int g = min(GROUP < kSdBlock ? n * NN + k : n >> bpg_shift, groups - 1);
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 const float4 v = *reinterpret_cast<const float4 *>(scales + g * S::kScaleRow + 4 * q);
@@ -233,7 +200,7 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
 #pragma unroll
                 for (int q = 0; q < NQ; ++q) acc[q] = __builtin_amdgcn_mfma_f32_4x4x4f16(a[q], b, acc[q], 4, P, 0);
                 if constexpr (GROUP < kSdBlock && 4 * (P + 1) % GROUP == 0)
-                    close(it, 4 * (P + 1) / GROUP - 1, s.norms[4 * (P + 1) / GROUP - 1], xs[4 * (P + 1) / GROUP - 1]);
+                    close(n * NN + 4 * (P + 1) / GROUP - 1, s.norms[4 * (P + 1) / GROUP - 1], xs[4 * (P + 1) / GROUP - 1]);
             });
             // pins the dword's products and sums before the next dword's reads
 #pragma unroll
@@ -243,39 +210,32 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
             __builtin_amdgcn_sched_barrier(0);
         });
         if constexpr (GROUP >= kSdBlock) {
-            if ((n & (bpg - 1)) == bpg - 1) close(it, 0, s.norms[0], xs[0]);
+            if ((n & (bpg - 1)) == bpg - 1) close(n >> bpg_shift, s.norms[0], xs[0]);
         }
         load_rest(s, ahead);
-        if constexpr (KS > 1) {
-            if ((n & (bpg - 1)) == bpg - 1) __syncthreads();
-        }
     };
     int n = 0;
-    for (; n + 2 <= count; n += 2) {
+    for (; n + 2 <= blocks; n += 2) {
         block_step(std::integral_constant<int, 0>{}, n);
         block_step(std::integral_constant<int, 1>{}, n + 1);
     }
-    if (n < count) block_step(std::integral_constant<int, 0>{}, n);
-    if constexpr (FIRST) {
-        if constexpr (KS > 1) add_parked(rounds - 1);
-        const int row = tile * kRowsPerBlock + r;
-        const size_t ys = J.ystride ? J.ystride : J.rows;
-        if (row < J.rows) {
+    if (n < blocks) block_step(std::integral_constant<int, 0>{}, n);
+    const int row = tile * kRowsPerBlock + r;
+    const size_t ys = J.ystride ? J.ystride : J.rows;
+    if (row < J.rows) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
-                if (b < nb) ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0 + b) * ys + row] = value[b];
-        }
+        for (int b = 0; b < NB; ++b)
+            if (b < nb) ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0 + b) * ys + row] = value[b];
     }
 }
 
-template <int GROUP, int NB, int KS>
-__global__ __launch_bounds__(kRowsPerBlock *KS, 2) void sdot_batch_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
+template <int GROUP, int NB>
+__global__ __launch_bounds__(kRowsPerBlock, 2) void sdot_batch_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
                                                                         int njobs, SdotGeom geom) {
     using S = SdShape<GROUP, NB>;
     extern __shared__ __attribute__((aligned(16))) uint32_t sd_lds[];
     uint32_t *table = sd_lds;
-    float *park = reinterpret_cast<float *>(sd_lds + kSdPairTable);
-    float *scales = park + SdPark<GROUP, NB, KS>::kTotal;  // [groups][kScaleRow]
+    float *scales = reinterpret_cast<float *>(sd_lds + kSdPairTable);  // [groups][kScaleRow]
     const int blk = blockIdx.x, b0 = blockIdx.y * NB;
     SdotJob J = job0;
     if (njobs > 0) {
@@ -295,31 +255,32 @@ __global__ __launch_bounds__(kRowsPerBlock *KS, 2) void sdot_batch_kernel(SdotJo
         const int c = static_cast<int8_t>((geom.cent[code >> 2] >> (8 * (code & 3))) & 0xFFu);
         return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(c))));
     };
-    for (int i = threadIdx.x; i < kSdPairTable / 4; i += kRowsPerBlock * KS) {  // 16 stores of 4 columns per entry
-        const int e = i >> 4;
-        const uint32_t v = half_of(e & 15) | half_of(e >> 4) << 16;
-        reinterpret_cast<u32x4 *>(table)[i] = u32x4{v, v, v, v};
+    // 16 stores of 4 columns per entry: the thread's entries share the low code, and the high one is the step
+    uint32_t lo = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lo = static_cast<int>(threadIdx.x >> 4) == i ? half_of(i) : lo;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const uint32_t v = lo | half_of(k) << 16;
+        reinterpret_cast<u32x4 *>(table)[threadIdx.x + k * kRowsPerBlock] = u32x4{v, v, v, v};
     }
     const int nb = min(NB, J.batch - b0);
-    for (int i = threadIdx.x; i < geom.groups * S::kScaleRow; i += kRowsPerBlock * KS) {
+    for (int i = threadIdx.x; i < geom.groups * S::kScaleRow; i += kRowsPerBlock) {
         const int g = i / S::kScaleRow, b = i % S::kScaleRow;
         scales[i] = b < nb ? J.xs[static_cast<size_t>(b0 + b) * geom.groups + g] : 0.0f;
     }
     __syncthreads();
-    const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kRowsPerBlock) : 0;
-    if (part == 0) sd_rows<GROUP, NB, KS, true>(J, geom, table, park, scales, blk, b0, 0);
-    else sd_rows<GROUP, NB, KS, KS == 1>(J, geom, table, park, scales, blk, b0, part);
+    sd_rows<GROUP, NB>(J, geom, table, scales, blk, b0);
 }
 
-template <int GROUP, int NB, int KS>
+template <int GROUP, int NB>
 bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                      hipStream_t s) {
     using S = SdShape<GROUP, NB>;
-    const size_t lds = (static_cast<size_t>(kSdPairTable) + SdPark<GROUP, NB, KS>::kTotal +
-                        static_cast<size_t>(g.groups) * S::kScaleRow) * 4;
+    const size_t lds = (static_cast<size_t>(kSdPairTable) + static_cast<size_t>(g.groups) * S::kScaleRow) * 4;
     if (lds > kSdMaxLds) return false;
-    const dim3 grid(blocks, (batch + NB - 1) / NB), block(kRowsPerBlock * KS);
-    hipLaunchKernelGGL((sdot_batch_kernel<GROUP, NB, KS>), grid, block, lds, s, job0, jobs, njobs, g);
+    const dim3 grid(blocks, (batch + NB - 1) / NB), block(kRowsPerBlock);
+    hipLaunchKernelGGL((sdot_batch_kernel<GROUP, NB>), grid, block, lds, s, job0, jobs, njobs, g);
     ND_HIP(hipGetLastError());
     return true;
 }
@@ -327,13 +288,9 @@ bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs
 template <int GROUP>
 bool sd_launch_group(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                      hipStream_t s) {
-    const int tiles = (batch + 15) / 16, rows = (batch + tiles - 1) / tiles;  // batch rows of a tile, all alike
+    const int tiles = (batch + 11) / 12, rows = (batch + tiles - 1) / tiles;  // batch rows of a tile, all alike
     auto go = [&](auto nb) {
-        constexpr int NB = decltype(nb)::value;
-        // up to one workgroup per CU: two parts over K
-        if (NB <= 8 && static_cast<long>(blocks) * tiles <= 256 && g.groups >= 4)
-            return sd_launch_shape<GROUP, NB, NB <= 8 ? 2 : 1>(g, job0, jobs, njobs, blocks, batch, s);
-        return sd_launch_shape<GROUP, NB, 1>(g, job0, jobs, njobs, blocks, batch, s);
+        return sd_launch_shape<GROUP, decltype(nb)::value>(g, job0, jobs, njobs, blocks, batch, s);
     };
     if (rows <= 2) return go(std::integral_constant<int, 2>{});
     if (rows <= 3) return go(std::integral_constant<int, 3>{});
@@ -341,8 +298,7 @@ bool sd_launch_group(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs
     if (rows <= 5) return go(std::integral_constant<int, 5>{});
     if (rows <= 6) return go(std::integral_constant<int, 6>{});
     if (rows <= 8) return go(std::integral_constant<int, 8>{});
-    if (rows <= 12) return go(std::integral_constant<int, 12>{});
-    return go(std::integral_constant<int, 16>{});
+    return go(std::integral_constant<int, 12>{});
 }
 
 }  // namespace

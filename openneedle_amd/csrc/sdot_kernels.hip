@@ -810,11 +810,15 @@ void launch_sdot_row(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs
 // DOTS the int32 group dots themselves are stored (dots[b][row][g]).
 // ---------------------------------------------------------------------------
 constexpr int kQuadMaxLds = 160 * 1024;
-// LDS rows of activations carry padding dwords, so that the batch rows that one
-// read touches lie in different banks (unpadded, every row of a power-of-two
-// width starts in the same bank: the 16-row reads of tile16 serialised
-// 16-fold).
+// LDS rows of activations carry four padding dwords, so that the batch rows
+// that one read touches lie in different banks (unpadded, the rows of a width
+// that is a multiple of 256 all start in the same bank). 32 x CQ4 4096 x 4096
+// g64 at batch 8 on the quad kernel 92 -> 77 us, at batch 16 on tile16 102 ->
+// 99 us. tile16's 16-byte reads of 2-bit matrices measured no faster with it
+// (g128, batch 16: 59 us without).
 constexpr int kRowPad = 4;
+template <int KIND>
+constexpr int kTile16Pad = KIND == kNib ? kRowPad : 0;
 
 template <int KIND, int GROUP, int NQ, bool DOTS>
 __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
@@ -1034,11 +1038,11 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     const int groups = geom.groups;
     const int dev = geom.windows * kWindow;
     const int qdw = dev / 4;
-    const int ldw = qdw + kRowPad;  // dwords of a batch row in LDS
+    const int ldw = qdw + kTile16Pad<KIND>;  // dwords of a batch row in LDS
     const int b0 = static_cast<int>(blockIdx.y) * TB;
     const int nb = min(TB, J.batch - b0);
     uint32_t *lq = t16_lds;
-    float *lxs = reinterpret_cast<float *>(t16_lds + TB * ldw);  // [groups][16]
+    float *lxs = reinterpret_cast<float *>(t16_lds + TB * ldw);
     const uint32_t cent[4] = {geom.cent[0], geom.cent[1], geom.cent[2], geom.cent[3]};
     const float cs = geom.centroid_scale;
     const __amdgpu_buffer_rsrc_t codes =
@@ -1071,10 +1075,10 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     // stage the tile's activation rows and group scales (rows past the batch as zeros)
     const u32x4 *q4 = reinterpret_cast<const u32x4 *>(J.q) + static_cast<size_t>(b0) * (qdw / 4);
     for (int i = threadIdx.x; i < TB * qdw / 4; i += kRowsPerBlock)
-        reinterpret_cast<u32x4 *>(lq)[i + i / (qdw / 4) * (kRowPad / 4)] =
+        reinterpret_cast<u32x4 *>(lq)[i + i / (qdw / 4) * (kTile16Pad<KIND> / 4)] =
             i / (qdw / 4) < nb ? q4[i] : u32x4{0, 0, 0, 0};
     for (int i = threadIdx.x; i < TB * groups; i += kRowsPerBlock)
-        lxs[i % groups * TB + i / groups] = i / groups < nb ? J.xs[static_cast<size_t>(b0) * groups + i] : 0.0f;
+        lxs[i] = i / groups < nb ? J.xs[static_cast<size_t>(b0) * groups + i] : 0.0f;
     __syncthreads();
     float value[4][4];  // [m][r]: weight row wrow + 16 m + jr, batch row 4 t + r
 #pragma unroll
@@ -1085,8 +1089,9 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
 #pragma unroll
     for (int m = 0; m < 4; ++m) acc[m] = v4i{0, 0, 0, 0};
     const uint32_t *qrow = lq + jr * ldw + 2 * H * t;  // batch row jr: the activation dwords of code dword t
-    const float *xrow = lxs + 4 * t;               // scales of batch rows 4t .. 4t + 3
-    auto read_a = [&](long (&a)[H], int c) {
+    const float *xrow = lxs + 4 * t * groups;      // scales of batch rows 4t .. 4t + 3
+    auto chunk = [&](const Tile16Slot &sl, int c, bool closes) {
+        long a[H];
         if constexpr (KIND == kNib) {
             const auto q2 = *reinterpret_cast<const uint32_t __attribute__((ext_vector_type(2))) *>(qrow + c * 8);
             a[0] = static_cast<long>(q2[0]) | (static_cast<long>(q2[1]) << 32);
@@ -1095,13 +1100,6 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
             a[0] = static_cast<long>(q4v.x) | (static_cast<long>(q4v.y) << 32);
             a[1] = static_cast<long>(q4v.z) | (static_cast<long>(q4v.w) << 32);
         }
-    };
-    long ahead[2][H];
-    read_a(ahead[0], 0);
-    // kc: c modulo 2; the next chunk's activations are read before this one's products (past the end: the last's)
-    auto chunk = [&](const Tile16Slot &sl, int c, int kc, bool closes) {
-        const long (&a)[H] = ahead[kc];
-        read_a(ahead[kc ^ 1], min(c + 1, nch - 1));
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             uint32_t wq[2 * H];  // the centroid dwords of code dword t, in activation-dword order
@@ -1130,8 +1128,9 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
                             dots[(static_cast<size_t>(b0 + 4 * t + r) * J.rows + row) * groups + g] = acc[m][r];
                 }
             } else {
-                const float4 xs4 = *reinterpret_cast<const float4 *>(xrow + g * TB);
-                const float xsb[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
+                float xsb[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) xsb[r] = xrow[r * groups + g];
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
                     const float ns = h2f(sl.norm[m]) * cs;  // sdot.cpp:43-44
@@ -1148,13 +1147,13 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_tile16_kernel(SdotJob job0
     for (; c0 + kRowRing <= nch; c0 += kRowRing) {
 #pragma unroll
         for (int k = 0; k < kRowRing; ++k) {
-            chunk(ring[k], c0 + k, k & 1, (k + 1) % CPG == 0);
+            chunk(ring[k], c0 + k, (k + 1) % CPG == 0);
             load(ring[k], min(c0 + k + kRowRing, nch - 1), (k + 1) % CPG == 0);
         }
     }
 #pragma unroll
     for (int k = 0; k < kRowRing; ++k)
-        if (c0 + k < nch) chunk(ring[k], c0 + k, k & 1, (k + 1) % CPG == 0);
+        if (c0 + k < nch) chunk(ring[k], c0 + k, (k + 1) % CPG == 0);
     if constexpr (!DOTS) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -1172,7 +1171,7 @@ template <int KIND, bool DOTS>
 bool launch_sdot_tile16(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                         int32_t *dots, hipStream_t s) {
     const int dev = g.windows * kWindow;
-    const size_t lds = static_cast<size_t>(16) * (dev + 4 * kRowPad) + static_cast<size_t>(16) * g.groups * 4;
+    const size_t lds = static_cast<size_t>(16) * (dev + 4 * kTile16Pad<KIND>) + static_cast<size_t>(16) * g.groups * 4;
     if (g.group < (KIND == kNib ? 32 : 64) || g.group > kWindow || lds > kQuadMaxLds) return false;
     dim3 grid(blocks, (batch + 15) / 16), block(kRowsPerBlock);
     switch (g.group) {
@@ -1838,17 +1837,21 @@ static bool tile16_wanted(int batch) {
     return batch > 8;
 }
 
-// The fp16 batch kernel (sdot_batch.hip) from 2 rows up (NEEDLE2_GPU_INT8_BATCH
-// "always" / "never"; an override of one of the kernels it stands before
-// leaves it out).
-static bool batch_wanted() {
+// The fp16 batch kernel (sdot_batch.hip): 4-bit codes in groups of 32 or 64, 2
+// .. 12 rows (NEEDLE2_GPU_INT8_BATCH "always" / "never"; an override of one of
+// the kernels it stands before leaves it out). 32 x CQ4 4096 x 4096 against
+// the quad kernel (tile16 at 12 rows): g32 at 2 / 4 / 8 / 12 rows 63 / 65 / 83
+// / 97 against 69 / 74 / 100 / 105 us, g64 60 / 61 / 79 / 91 against 63 / 65 /
+// 81 / 104; g128 56 / 59 / 74 against 57 / 56 / 76; at 16 rows its 4 x 4 x 4
+// products take longer than tile16 (g32 116 against 110, g128 108 against 98).
+static bool batch_wanted(const SdotGeom &g, int batch) {
     const char *mode = std::getenv("NEEDLE2_GPU_INT8_BATCH");
     if (mode && (std::strcmp(mode, "always") == 0 || std::strcmp(mode, "never") == 0)) return mode[0] == 'a';
     for (const char *name : {"NEEDLE2_GPU_INT8_TILE16", "NEEDLE2_GPU_INT8_QUAD", "NEEDLE2_GPU_INT8_MFMA"}) {
         const char *other = std::getenv(name);
         if (other && (std::strcmp(other, "always") == 0 || std::strcmp(other, "never") == 0)) return false;
     }
-    return true;
+    return g.group <= 64 && batch <= 12;
 }
 
 // The K split for small matrices (NEEDLE2_GPU_INT8_KSPLIT "always" / "never") and, within it, the 16 x 16
@@ -1933,7 +1936,7 @@ void launch_sdot_gemv(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
         else launch_sdot_row<kCrumb, false>(g, job0, jobs, njobs, blocks, nullptr, s);
         return;
     }
-    if (batch >= 2 && batch_wanted() && launch_sdot_batch(g, job0, jobs, njobs, blocks, batch, s)) return;
+    if (batch >= 2 && batch_wanted(g, batch) && launch_sdot_batch(g, job0, jobs, njobs, blocks, batch, s)) return;
     if (!mfma_forced && tile16_wanted(batch)) {
         const bool done = g.kind == kNib ? launch_sdot_tile16<kNib, false>(g, job0, jobs, njobs, blocks, batch, nullptr, s)
                                          : launch_sdot_tile16<kCrumb, false>(g, job0, jobs, njobs, blocks, batch, nullptr, s);
