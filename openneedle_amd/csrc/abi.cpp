@@ -186,7 +186,7 @@ void CqHandle::gemv(const uint4 *codes, const uint16_t *norms, int rows, int n_p
 void matrix_gemv(const Matrix &m, Staging &st, const uint4 *codes, const uint16_t *norms, int rows, int n_pad,
                  const float *d_x, float *d_y, int batch, hipStream_t s) {
     const float *act = d_x;
-    const GemvPath path = gemv_path(m.group, m.in, m.dev, batch);
+    const GemvPath path = gemv_path(m.kind, m.group, m.in, m.dev, n_pad / kRowsPerBlock, batch);
     if (!path.raw) {
         st.rot.reserve(size_t(batch) * m.dev);
         if (gemv_prepass(m.group))
@@ -300,7 +300,7 @@ void CqHandle::linear_host(const float *x, float *y, int batch) {
     // workgroup (one row, groups of 128 / 256) reads a device copy. y is written once
     // per value, straight into the pinned buffer. Each host-device copy saved
     // is ~7 us of a CQ4 8192 x 8192 call (80 -> 66 us).
-    const bool x_direct = m.in <= 2 * kWindow || !gemv_path(m.group, m.in, m.dev, batch).raw;
+    const bool x_direct = m.in <= 2 * kWindow || !gemv_path(m.kind, m.group, m.in, m.dev, m.n_pad / kRowsPerBlock, batch).raw;
     const float *dx = st.hx.p;
     if (!x_direct) {
         st.x.reserve(nx);
@@ -486,7 +486,9 @@ static void plan_upload(Plan &p) {
     if (!p.sdot) {
         p.rot.reserve(size_t(p.count) * p.batch * m.dev);
         std::vector<CqJob> jobs(p.count);
-        p.path = gemv_path(m.group, m.in, m.dev, p.batch);
+        int blocks = 0;
+        for (const CqHandle *h : p.cq) blocks += h->m.n_pad / kRowsPerBlock;
+        p.path = gemv_path(m.kind, m.group, m.in, m.dev, blocks, p.batch);
         for (int i = 0; i < p.count; ++i) {
             const Matrix &mi = p.cq[i]->m;
             const float *act = p.path.raw ? p.xs_in[i] : p.rot.p + size_t(i) * p.batch * m.dev;
@@ -652,7 +654,7 @@ static void linear_many(const std::vector<CqHandle *> &hs, const float *x, float
     ND_HIP(hipMemcpyAsync(st.x.p, st.hx.p, size_t(m0.in) * sizeof(float), hipMemcpyHostToDevice, s));
     // the one transform: the shared rotated x, unless the GEMV fuses the FWHT into its table build
     const float *act = st.x.p;
-    const GemvPath path = gemv_path(m0.group, m0.in, m0.dev, 1);
+    const GemvPath path = gemv_path(m0.kind, m0.group, m0.in, m0.dev, 0, 1);
     if (!path.raw) {
         st.rot.reserve(m0.dev);
         if (gemv_prepass(m0.group)) launch_rot_many(st.x.p, nullptr, 1, 1, m0.in, m0.dev, m0.group, m0.scale, st.rot.p, s);

@@ -1066,7 +1066,7 @@ __device__ __forceinline__ void quad_add_parked(const float *P, int r, float &su
 
 // XF: J.act is the raw input ([batch][in]), transformed here (quad_act_x),
 // instead of the pre-pass output ([batch][dev]).
-template <int KIND, int GROUP, int QUAD, bool XF>
+template <int KIND, int GROUP, int QUAD, bool XF, bool PAIRS = false>
 __device__ __forceinline__ void quad_rows(const CqJob &J, const CqGeom &geom, float (*T)[QuadShape<KIND, GROUP>::kFloats],
                                           float (*P)[(kQuads - 1) * QuadShape<KIND, GROUP>::kGroups * kRowsPerBlock],
                                           int blk) {
@@ -1088,7 +1088,69 @@ __device__ __forceinline__ void quad_rows(const CqJob &J, const CqGeom &geom, fl
     for (int i = 0; i < 16; ++i) lut[i] = geom.lut[i];
 
     const int stride = XF ? geom.in : dev;
-    for (int b = 0; b < batch; ++b) {
+    // Two activation rows per pass over the codes (the reference pairs tokens,
+    // cq.cpp:110-152): each window's chunks are loaded once and feed both rows'
+    // tables, row b0 then row b0 + 1 (passes alternate the table and park
+    // buffers; quarter 0 adds a pass's parked groups at the next pass, before
+    // that row's next window). Per row the order of every operation is that of
+    // the one-row loop below, so the outputs are the same bits.
+    int b0 = 0;
+    for (; PAIRS && b0 + 1 < batch; b0 += 2) {
+        const __amdgpu_buffer_rsrc_t rot0 =
+            buffer_rsrc(J.act + static_cast<size_t>(b0) * stride, static_cast<uint32_t>(stride) * 4u);
+        const __amdgpu_buffer_rsrc_t rot1 =
+            buffer_rsrc(J.act + static_cast<size_t>(b0 + 1) * stride, static_cast<uint32_t>(stride) * 4u);
+        // activations of pass q = 2 w + row (past the last window: zeros)
+        auto act = [&](int q) {
+            const __amdgpu_buffer_rsrc_t &rt = (q & 1) ? rot1 : rot0;
+            if constexpr (XF) return quad_act_x<KIND, GROUP>(rt, q >> 1, r, geom.scale);
+            else return quad_act<KIND>(rt, q >> 1, r);
+        };
+        QuadState<KIND, GROUP> cur, nxt;
+        float2 xr = act(0);
+        quad_load<KIND, GROUP>(cur, codes, norms, 0, QUAD, r);
+        quad_load<KIND, GROUP>(nxt, codes, norms, 1, QUAD, r);
+        __syncthreads();  // the previous rows finished with T[0] and P
+        quad_build<KIND, GROUP>(T[0], lut, xr, QUAD, r);
+        xr = act(1);
+        __syncthreads();
+        float sum[2] = {0.0f, 0.0f}, gd = 0.0f;
+        // pass (w, row): table T[row], parked P[row]; at its start quarter 0 adds
+        // the previous pass's parked groups (the other row's, same or previous
+        // window) into that row's sum
+        auto pass = [&](auto rowc, QuadState<KIND, GROUP> &st, int w) {
+            constexpr int row = decltype(rowc)::value;
+            if (QUAD == 0 && (row == 1 || w > 0))
+                quad_add_parked<KIND, GROUP>(P[row ^ 1], r, sum[row ^ 1], row == 1 ? w : w - 1, groups);
+            quad_compute<KIND, GROUP, QUAD, row == 1>(st, T[row], P[row], r, mask, sum[row], gd, w, groups, codes,
+                                                      norms);
+            const int q = 2 * w + row;
+            quad_build<KIND, GROUP>(T[row ^ 1], lut, xr, QUAD, r);
+            xr = act(q + 2);
+            __syncthreads();
+        };
+        const int pairs = windows / 2;
+        for (int it = 0; it < pairs; ++it) {
+            const int w = 2 * it;
+            pass(std::integral_constant<int, 0>{}, cur, w);
+            pass(std::integral_constant<int, 1>{}, cur, w);
+            pass(std::integral_constant<int, 0>{}, nxt, w + 1);
+            pass(std::integral_constant<int, 1>{}, nxt, w + 1);
+        }
+        if (windows & 1) {
+            const int w = windows - 1;
+            pass(std::integral_constant<int, 0>{}, cur, w);
+            pass(std::integral_constant<int, 1>{}, cur, w);
+        }
+        if (QUAD == 0) {
+            quad_add_parked<KIND, GROUP>(P[1], r, sum[1], windows - 1, groups);
+            if (row < rows) {
+                ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0) * rows + row] = sum[0];
+                ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0 + 1) * rows + row] = sum[1];
+            }
+        }
+    }
+    for (int b = b0; b < batch; ++b) {
         const __amdgpu_buffer_rsrc_t rot =
             buffer_rsrc(J.act + static_cast<size_t>(b) * stride, static_cast<uint32_t>(stride) * 4u);
         auto act = [&](int w) {
@@ -1169,6 +1231,39 @@ __global__ __launch_bounds__(kQuadThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
 }
 
+// The quarter GEMV for two rows: both over one pass of the codes (each chunk
+// loaded once). One workgroup per CU (128 VGPRs per lane: the pair loop holds
+// both rows' state and the two tables' pipelines). 16 x CQ4 8192^2 g32: 203 ->
+// 181 us against one row per pass; the batch kernel takes 247 where this one
+// takes 221 (another box), and less from three rows on.
+template <int KIND, int GROUP, bool XF>
+__global__ __launch_bounds__(kQuadThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void cq_gemv_quad_pair_kernel(
+    CqJob job0, const CqJob *__restrict__ jobs, int njobs, CqGeom geom) {
+    using Q = QuadShape<KIND, GROUP>;
+    __shared__ __attribute__((aligned(16))) float T[2][Q::kFloats];
+    __shared__ float P[2][(kQuads - 1) * Q::kGroups * kRowsPerBlock];
+    const int blk = blockIdx.x;
+    CqJob J = job0;
+    if (njobs > 0) {
+        const ND_CONST CqJob *cj = (const ND_CONST CqJob *)(jobs);
+        const int j = find_job(cj, njobs, blk);
+        J.codes = cj[j].codes;
+        J.norms = cj[j].norms;
+        J.act = cj[j].act;
+        J.y = cj[j].y;
+        J.rows = cj[j].rows;
+        J.n_pad = cj[j].n_pad;
+        J.block_begin = cj[j].block_begin;
+        J.batch = cj[j].batch;
+    }
+    switch (__builtin_amdgcn_readfirstlane(threadIdx.x / kRowsPerBlock)) {
+    case 0: quad_rows<KIND, GROUP, 0, XF, true>(J, geom, T, P, blk); break;
+    case 1: quad_rows<KIND, GROUP, 1, XF, true>(J, geom, T, P, blk); break;
+    case 2: quad_rows<KIND, GROUP, 2, XF, true>(J, geom, T, P, blk); break;
+    default: quad_rows<KIND, GROUP, 3, XF, true>(J, geom, T, P, blk); break;
+    }
+}
+
 // Activation pre-pass of the quarter and batch GEMVs: rot[v][0..dev) = per-group FWHT
 // of zero-padded x (the reference's transform, cq.cpp:153-156, identical
 // butterflies), for nvec = count * batch vectors at once: vector v is row
@@ -1187,9 +1282,28 @@ __global__ __launch_bounds__(kRowsPerBlock) void rot_many_kernel(const float *__
     if (p < dev) rot[static_cast<size_t>(v) * dev + p] = x[0];
 }
 
+// NEEDLE2_GPU_FP32_PAIRS=never: batches run one row per pass over the codes.
+static bool one_row_forced() {
+    const char *mode = std::getenv("NEEDLE2_GPU_FP32_PAIRS");
+    return mode && std::strcmp(mode, "never") == 0;
+}
+
 template <int KIND, bool XF>
-void launch_gemv_kind(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, hipStream_t s) {
+void launch_gemv_kind(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, int batch,
+                      hipStream_t s) {
     dim3 grid(blocks), block(kRowsPerBlock), split(kSplitThreads), quad(kQuadThreads);
+    if constexpr (KIND == kNib) {  // (2-bit: LDS-bound, and one workgroup per CU runs pairs slower: 132 -> 183 us)
+        if (g.group <= 64 && batch >= 2 && !one_row_forced()) {
+            switch (g.group) {
+            case 8: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 8, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
+            case 16: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 16, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
+            case 32: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 32, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
+            default: hipLaunchKernelGGL((cq_gemv_quad_pair_kernel<KIND, 64, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
+            }
+            ND_HIP(hipGetLastError());
+            return;
+        }
+    }
     switch (g.group > kWindow ? 0 : g.group) {
     case 8: hipLaunchKernelGGL((cq_gemv_quad_kernel<KIND, 8, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
     case 16: hipLaunchKernelGGL((cq_gemv_quad_kernel<KIND, 16, XF>), grid, quad, 0, s, job0, jobs, njobs, g); break;
@@ -1361,12 +1475,17 @@ static bool gemv_quad_takes_x(int group, int in) {
     return in <= 2 * kWindow;
 }
 
-// Batches run the batch kernel (NEEDLE2_GPU_FP32_PAIRS=never: one row per
-// pass over the codes). Its buffer resource spans eight rows, which must stay
-// under 2^32 bytes.
-GemvPath gemv_path(int group, int in, int dev, int batch) {
-    const char *mode = std::getenv("NEEDLE2_GPU_FP32_PAIRS");
-    const bool batched = batch >= 2 && dev <= 1 << 26 && !(mode && std::strcmp(mode, "never") == 0);
+// The batch kernel from four rows on, and from three except for 2-bit groups
+// of up to 64 (8 x 2048 x 4000: 52.0 against 50.5 us one row per pass; CQ4 g32
+// 57.8 against 72.0 in pairs). Two rows take it only for 4-bit groups above 64
+// and 32 row tiles or more (8 x 2048 x 4000 g128: 50.9 against 58.6 us; 2048 x
+// 512 11.3 against 8.8), the rest the pair kernel or one row per pass (CQ4 g32
+// 52.0 against 48.8, CQ2 g64 47.8 against 35.8). Its buffer resource spans
+// eight rows, which must stay under 2^32 bytes.
+GemvPath gemv_path(int kind, int group, int in, int dev, int blocks, int batch) {
+    const bool enough = batch >= 4 || (batch == 3 && !(kind == kCrumb && group <= 64)) ||
+                        (batch == 2 && kind == kNib && group > 64 && blocks >= 32);
+    const bool batched = enough && dev <= 1 << 26 && !one_row_forced();
     return {batched, gemv_quad_takes_x(group, in) || (gemv_fuses_fwht(group) && !batched)};
 }
 
@@ -1378,12 +1497,12 @@ void launch_cq_gemv(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int n
         return;
     }
     if (path.raw && g.group <= 64) {
-        if (g.kind == kNib) launch_gemv_kind<kNib, true>(g, job0, jobs, njobs, blocks, s);
-        else launch_gemv_kind<kCrumb, true>(g, job0, jobs, njobs, blocks, s);
+        if (g.kind == kNib) launch_gemv_kind<kNib, true>(g, job0, jobs, njobs, blocks, batch, s);
+        else launch_gemv_kind<kCrumb, true>(g, job0, jobs, njobs, blocks, batch, s);
         return;
     }
-    if (g.kind == kNib) launch_gemv_kind<kNib, false>(g, job0, jobs, njobs, blocks, s);
-    else launch_gemv_kind<kCrumb, false>(g, job0, jobs, njobs, blocks, s);
+    if (g.kind == kNib) launch_gemv_kind<kNib, false>(g, job0, jobs, njobs, blocks, batch, s);
+    else launch_gemv_kind<kCrumb, false>(g, job0, jobs, njobs, blocks, batch, s);
 }
 
 void launch_gather_rows(const uint4 *codes, const uint16_t *norms, int rows, int chunks, int groups,

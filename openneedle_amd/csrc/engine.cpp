@@ -68,9 +68,12 @@ struct Mat {
 };
 
 // Row tiles of several CQ matrices that share one input, run as one GEMV
-// launch (matrices of one geometry) after at most one activation transform:
-// one job per piece, of one row for a single token (decode step) and of T
-// rows for a prompt chunk of T tokens. Both are bit-identical per token.
+// launch (matrices of one geometry) after at most one activation transform.
+// The job table holds `tokens` copies of the pieces, token-major, each over
+// its token's input row and into its token's output rows, so a launch over
+// the first n tokens runs n times the workgroups of one token; chunks above
+// kBatchTokens run the batch kernel over one job of T rows per piece instead.
+// Both are bit-identical per token.
 struct GemvGroup {
     struct Piece {
         const Matrix *m;
@@ -78,13 +81,17 @@ struct GemvGroup {
         float *y;         // receives the piece's whole row tiles, from tile first / 256
         int ystride;      // floats between consecutive tokens' outputs
     };
+    // Six row tiles a token (the released geometry's Q|K|V|gate) fill the chip
+    // at some 40 tokens, and the one-row kernels then take ~34 us at 256 tokens
+    // where the transform and the batch kernel take 24; at 32 tokens ~6 against 17.
+    static constexpr int kBatchTokens = 128;
     const Matrix *m0 = nullptr;
-    DevBuf<uint8_t> jobs;  // `pieces` jobs of a single token, then those of a chunk
+    DevBuf<uint8_t> jobs;  // per-token jobs, then the `pieces` jobs of a long chunk
     DevBuf<float> rot, big;
-    int pieces = 0, blocks = 0;  // jobs and row tiles of one launch
+    int pieces = 0, per_token = 0, max_tokens = 0;  // jobs and row tiles of one token
     const float *x = nullptr;
     CqJob job0{};
-    GemvPath one{}, many{};  // a single token's launch, a chunk's
+    GemvPath one{}, many{};  // per-token jobs, a long chunk's
 
     static bool compatible(const Matrix &a, const Matrix &b) {
         return a.in == b.in && a.bits == b.bits && a.group == b.group &&
@@ -95,26 +102,30 @@ struct GemvGroup {
     void build(const std::vector<Piece> &ps, const float *input, int tokens) {
         m0 = ps[0].m;
         x = input;
-        one = gemv_path(m0->group, m0->in, m0->dev, 1);
-        many = gemv_path(m0->group, m0->in, m0->dev, tokens);
-        many.batched = true;  // the pieces' outputs are strided, which the one-row kernels do not write
-        many.raw = many.raw && m0->group <= 64;
+        max_tokens = tokens;
+        one = gemv_path(m0->kind, m0->group, m0->in, m0->dev, 0, 1);
+        many = GemvPath{true, one.raw && m0->group <= 64};
         if (!one.raw || !many.raw) rot.reserve(size_t(m0->dev) * tokens);
         std::vector<CqJob> host;
-        for (const GemvPath &path : {one, many}) {
-            blocks = 0;
+        int blocks = 0;
+        auto add = [&](const GemvPath &path, int t) {
             for (const Piece &p : ps) {
                 ND_CHECK(compatible(*m0, *p.m), "internal: GEMV group of mixed geometry");
                 const int tile0 = p.first / kRowsPerBlock;
                 const int tile1 = (p.first + p.rows - 1) / kRowsPerBlock;
                 const int tiles = tile1 - tile0 + 1;
                 const int rows = std::min(tiles * kRowsPerBlock, p.m->out - tile0 * kRowsPerBlock);
+                const float *act = path.raw ? input + size_t(t) * m0->in : rot.p + size_t(t) * m0->dev;
                 host.push_back(CqJob{p.m->codes.p + size_t(tile0) * p.m->chunks * kRowsPerBlock,
-                                     p.m->norms.p + size_t(tile0) * p.m->groups * kRowsPerBlock,
-                                     path.raw ? input : rot.p, p.y, rows, tiles * kRowsPerBlock, blocks, 1, p.ystride});
+                                     p.m->norms.p + size_t(tile0) * p.m->groups * kRowsPerBlock, act,
+                                     p.y + size_t(t) * p.ystride, rows, tiles * kRowsPerBlock, blocks, 1, p.ystride});
                 blocks += tiles;
             }
-        }
+        };
+        for (int t = 0; t < tokens; ++t) add(one, t);
+        per_token = blocks / tokens;
+        blocks = 0;
+        add(many, 0);
         pieces = static_cast<int>(ps.size());
         job0 = host[0];
         jobs.reserve(host.size() * sizeof(CqJob));
@@ -122,16 +133,22 @@ struct GemvGroup {
     }
 
     void run(hipStream_t s, int tokens) {
-        const GemvPath &path = tokens > 1 ? many : one;
+        const bool batch = tokens > kBatchTokens;
+        const GemvPath &path = batch ? many : one;
         if (!path.raw) {
             if (gemv_prepass(m0->group))
                 launch_rot_many(x, nullptr, tokens, tokens, m0->in, m0->dev, m0->group, m0->scale, rot.p, s);
             else
                 m0->transform(x, m0->in, rot.p, tokens, big, s);
         }
-        const auto *table = reinterpret_cast<const CqJob *>(jobs.p) + (tokens > 1 ? pieces : 0);
-        const bool by_value = tokens == 1 && pieces == 1;
-        launch_cq_gemv(m0->geom(), job0, by_value ? nullptr : table, by_value ? 0 : pieces, blocks, tokens, path, s);
+        const auto *table = reinterpret_cast<const CqJob *>(jobs.p);
+        const int njobs = pieces * tokens;
+        if (batch)
+            launch_cq_gemv(m0->geom(), CqJob{}, table + size_t(pieces) * max_tokens, pieces, per_token, tokens, path, s);
+        else if (njobs > 1)
+            launch_cq_gemv(m0->geom(), CqJob{}, table, njobs, per_token * tokens, 1, path, s);
+        else
+            launch_cq_gemv(m0->geom(), job0, nullptr, 0, per_token, 1, path, s);
     }
 };
 

@@ -23,6 +23,8 @@
 //    codebook lookup reads a 256-entry table of code pairs (two fp16 values
 //    per byte of codes) from LDS, one private column per lane so the reads
 //    are conflict-free: 4 v_perm + 4 ds_read_b32 + 4 v_pk_mul_f16 per 8 codes.
+//    Tall tiles (256 x 128, tall_tiles): waves 0-3 each own 64 rows over the
+//    whole of K.
 //
 // 2-bit (CQ2, ternary) matrices are widened once to 4-bit device codes of the
 // same positions (widen_crumbs_kernel), so one kernel serves every width.
@@ -626,6 +628,10 @@ void launch_prefill_transform(const float *x, int m, int in, int padded, int dev
 
 namespace {
 
+// 256-row tiles where they save rounds of the 256 CUs: a tall tile's step takes
+// 0.91 us against 0.67 (1999 x 11008 x 4096, group 128: three rounds instead of
+// six, 262 -> 196 us with the transform); 512 x 8192 x 2048 fills one round
+// with low tiles and would leave half the CUs idle with tall ones.
 bool tall_tiles(int ntiles, int m) {
     const int low = (ntiles * ((m + kBM - 1) / kBM) + 255) / 256;
     const int tall = (ntiles * ((m + 2 * kBM - 1) / (2 * kBM)) + 255) / 256;

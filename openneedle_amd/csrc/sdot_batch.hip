@@ -79,6 +79,25 @@ __device__ __forceinline__ void sd_pairs(uint32_t (&v)[4], const uint32_t *table
             __builtin_amdgcn_perm(dword, lane4, 0x0c0c0400u + (static_cast<uint32_t>(k) << 8)));
 }
 
+// Entry e (a byte of codes, low nibble first): 16 stores of 4 columns. A
+// thread's entries share the low code, and the high one is the step (no
+// indexed read of the arguments).
+__device__ __forceinline__ void fill_pair_table(uint32_t *table, const SdotGeom &geom) {
+    auto half_of = [&](int code) {  // the code's int8 centroid as fp16
+        const int c = static_cast<int8_t>((geom.cent[code >> 2] >> (8 * (code & 3))) & 0xFFu);
+        return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(c))));
+    };
+    const int low = threadIdx.x >> 4;
+    uint32_t lo = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lo = low == i ? half_of(i) : lo;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const uint32_t v = lo | half_of(k) << 16;
+        reinterpret_cast<u32x4 *>(table)[threadIdx.x + k * kRowsPerBlock] = u32x4{v, v, v, v};
+    }
+}
+
 template <class F, int... I>
 __device__ __forceinline__ void sd_for_impl(F &&f, std::integer_sequence<int, I...>) {
     (f(std::integral_constant<int, I>{}), ...);
@@ -233,9 +252,9 @@ template <int GROUP, int NB>
 __global__ __launch_bounds__(kRowsPerBlock, 2) void sdot_batch_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
                                                                         int njobs, SdotGeom geom) {
     using S = SdShape<GROUP, NB>;
-    extern __shared__ __attribute__((aligned(16))) uint32_t sd_lds[];
-    uint32_t *table = sd_lds;
-    float *scales = reinterpret_cast<float *>(sd_lds + kSdPairTable);  // [groups][kScaleRow]
+    // (a static table: its address folds into the lookups)
+    __shared__ __attribute__((aligned(16))) uint32_t table[kSdPairTable];
+    extern __shared__ __attribute__((aligned(16))) float scales[];  // [groups][kScaleRow]
     const int blk = blockIdx.x, b0 = blockIdx.y * NB;
     SdotJob J = job0;
     if (njobs > 0) {
@@ -251,19 +270,7 @@ __global__ __launch_bounds__(kRowsPerBlock, 2) void sdot_batch_kernel(SdotJob jo
         J.batch = cj[j].batch;
         J.ystride = cj[j].ystride;
     }
-    auto half_of = [&](int code) {  // the code's int8 centroid as fp16
-        const int c = static_cast<int8_t>((geom.cent[code >> 2] >> (8 * (code & 3))) & 0xFFu);
-        return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(c))));
-    };
-    // 16 stores of 4 columns per entry: the thread's entries share the low code, and the high one is the step
-    uint32_t lo = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) lo = static_cast<int>(threadIdx.x >> 4) == i ? half_of(i) : lo;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const uint32_t v = lo | half_of(k) << 16;
-        reinterpret_cast<u32x4 *>(table)[threadIdx.x + k * kRowsPerBlock] = u32x4{v, v, v, v};
-    }
+    fill_pair_table(table, geom);
     const int nb = min(NB, J.batch - b0);
     for (int i = threadIdx.x; i < geom.groups * S::kScaleRow; i += kRowsPerBlock) {
         const int g = i / S::kScaleRow, b = i % S::kScaleRow;
@@ -277,8 +284,8 @@ template <int GROUP, int NB>
 bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                      hipStream_t s) {
     using S = SdShape<GROUP, NB>;
-    const size_t lds = (static_cast<size_t>(kSdPairTable) + static_cast<size_t>(g.groups) * S::kScaleRow) * 4;
-    if (lds > kSdMaxLds) return false;
+    const size_t lds = static_cast<size_t>(g.groups) * S::kScaleRow * 4;
+    if (lds + kSdPairTable * 4 > kSdMaxLds) return false;
     const dim3 grid(blocks, (batch + NB - 1) / NB), block(kRowsPerBlock);
     hipLaunchKernelGGL((sdot_batch_kernel<GROUP, NB>), grid, block, lds, s, job0, jobs, njobs, g);
     ND_HIP(hipGetLastError());

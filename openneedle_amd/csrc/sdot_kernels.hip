@@ -1840,10 +1840,10 @@ static bool tile16_wanted(int batch) {
 // The fp16 batch kernel (sdot_batch.hip): 4-bit codes in groups of 32 or 64, 2
 // .. 12 rows (NEEDLE2_GPU_INT8_BATCH "always" / "never"; an override of one of
 // the kernels it stands before leaves it out). 32 x CQ4 4096 x 4096 against
-// the quad kernel (tile16 at 12 rows): g32 at 2 / 4 / 8 / 12 rows 63 / 65 / 83
-// / 97 against 69 / 74 / 100 / 105 us, g64 60 / 61 / 79 / 91 against 63 / 65 /
-// 81 / 104; g128 56 / 59 / 74 against 57 / 56 / 76; at 16 rows its 4 x 4 x 4
-// products take longer than tile16 (g32 116 against 110, g128 108 against 98).
+// the quad kernel (tile16 at 12 rows): g32 at 2 / 4 / 8 / 12 rows 55 / 63 / 77
+// / 92 against 68 / 73 / 95 / 104 us, g64 52 / 55 / 73 / 90 against 61 / 62 /
+// 80 / 104; g128 56 / 59 / 74 against 57 / 56 / 76 (another build); at 16 rows
+// its 4 x 4 x 4 products take longer than tile16 (116 against 110).
 static bool batch_wanted(const SdotGeom &g, int batch) {
     const char *mode = std::getenv("NEEDLE2_GPU_INT8_BATCH");
     if (mode && (std::strcmp(mode, "always") == 0 || std::strcmp(mode, "never") == 0)) return mode[0] == 'a';
