@@ -44,19 +44,21 @@ static void check_layer(const KvHandle &kv, int layer) {
 // Splits of the slot range: enough (sequence, kv head, split) blocks for two
 // per CU, never a split shorter than one 256-slot tile. With that many
 // (sequence, kv head) pairs already (a large decode batch) there is one split
-// and no merge pass, nor where the other tiles of a range cost a block less
-// than the merge pass (about 2.5 us: 4 x 8 kv heads x 300 slots of 128, 2
+// and no merge pass, nor on the matrix kernel (whose sums are short enough for
+// it: its error is below the vector kernel's over any number of splits) where
+// the other tiles of a range cost a block less than the merge pass (about 2.5 us: 4 x 8 kv heads x 300 slots of 128, 2
 // heads each, 10.2 -> 8.0 us with one split, 7 x 4 x 777 slots of 32 8.0 ->
 // 6.8 us). A block alone walks a tile in 0.3 us + 2.7 us per 1024 head
 // values (one kv head x 8 heads x 8192 slots of 128: 97 us in one split).
-static int auto_splits(int pairs, int length, int values) {
+static int auto_splits(int pairs, int length, int group, int head_dim) {
     static const int cus = [] {  // queried once
         int dev = 0, n = 256;
         if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
         return n;
     }();
     const int tiles = (length + 255) / 256;
-    if ((tiles - 1) * (0.3 + 2.7 * values / 1024) < 2.5) return 1;
+    const bool matrix = group > 1 || head_dim == 128;
+    if (matrix && (tiles - 1) * (0.3 + 2.7 * group * head_dim / 1024) < 2.5) return 1;
     const int want = (2 * cus + pairs - 1) / pairs;
     return std::max(1, std::min(want, tiles));
 }
@@ -206,7 +208,7 @@ int needle2_gpu_attention_chained(void *h, int layer, const float *d_q, float *d
         ND_CHECK(d_q && d_out, "attention: null q or out");
         hipStream_t s = static_cast<hipStream_t>(stream);
         const int pairs = kv.seqs * kv.kvheads;
-        if (splits <= 0) splits = auto_splits(pairs, length, group * kv.head_dim);
+        if (splits <= 0) splits = auto_splits(pairs, length, group, kv.head_dim);
         const int tiles = std::max(1, (length + 255) / 256);
         splits = std::min(splits, tiles);
         const int per = (tiles + splits - 1) / splits * 256;  // whole tiles per split
