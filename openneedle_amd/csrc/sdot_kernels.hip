@@ -1838,20 +1838,24 @@ static bool tile16_wanted(int batch) {
 }
 
 // The fp16 batch kernel (sdot_batch.hip): 4-bit codes in groups of 32 or 64, 2
-// .. 12 rows (NEEDLE2_GPU_INT8_BATCH "always" / "never"; an override of one of
-// the kernels it stands before leaves it out). 32 x CQ4 4096 x 4096 against
-// the quad kernel (tile16 at 12 rows): g32 at 2 / 4 / 8 / 12 rows 55 / 63 / 77
-// / 92 against 68 / 73 / 95 / 104 us, g64 52 / 55 / 73 / 90 against 61 / 62 /
-// 80 / 104; g128 56 / 59 / 74 against 57 / 56 / 76 (another build); at 16 rows
-// its 4 x 4 x 4 products take longer than tile16 (116 against 110).
-static bool batch_wanted(const SdotGeom &g, int batch) {
+// .. 12 rows, or 128, 2 .. 8 rows (NEEDLE2_GPU_INT8_BATCH "always" / "never";
+// an override of one of the kernels it stands before leaves it out). 32 x CQ4
+// 4096 x 4096 against the quad kernel (tile16 at 12 rows): g32 at 2 / 4 / 8 /
+// 12 rows 55 / 63 / 77 / 92 against 68 / 73 / 95 / 104 us, g64 52 / 55 / 73 /
+// 90 against 61 / 62 / 80 / 104, g128 53 / 57 / 70 against 54 / 59 / 77. Its
+// table costs each workgroup some 2 us, so it takes 384 row tiles and, under
+// four rows, 8192 windows of them (g128: 24 x 5003 x 3000 at 3 / 5 rows 39.5 /
+// 44.4 against 36.2 / 48.1, 6 x 8000 x 2000 at 2 rows 20.7 against 18.0). At 16
+// rows its 4 x 4 x 4 products take longer than tile16 (116 against 110).
+static bool batch_wanted(const SdotGeom &g, int blocks, int batch) {
     const char *mode = std::getenv("NEEDLE2_GPU_INT8_BATCH");
     if (mode && (std::strcmp(mode, "always") == 0 || std::strcmp(mode, "never") == 0)) return mode[0] == 'a';
     for (const char *name : {"NEEDLE2_GPU_INT8_TILE16", "NEEDLE2_GPU_INT8_QUAD", "NEEDLE2_GPU_INT8_MFMA"}) {
         const char *other = std::getenv(name);
         if (other && (std::strcmp(other, "always") == 0 || std::strcmp(other, "never") == 0)) return false;
     }
-    return g.group <= 64 && batch <= 12;
+    if (blocks < 384 || (batch < 4 && static_cast<long>(blocks) * g.windows < 8192)) return false;
+    return g.group <= 128 && batch <= (g.group <= 64 ? 12 : 8);
 }
 
 // The K split for small matrices (NEEDLE2_GPU_INT8_KSPLIT "always" / "never") and, within it, the 16 x 16
@@ -1936,7 +1940,7 @@ void launch_sdot_gemv(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
         else launch_sdot_row<kCrumb, false>(g, job0, jobs, njobs, blocks, nullptr, s);
         return;
     }
-    if (batch >= 2 && batch_wanted(g, batch) && launch_sdot_batch(g, job0, jobs, njobs, blocks, batch, s)) return;
+    if (batch >= 2 && batch_wanted(g, blocks, batch) && launch_sdot_batch(g, job0, jobs, njobs, blocks, batch, s)) return;
     if (!mfma_forced && tile16_wanted(batch)) {
         const bool done = g.kind == kNib ? launch_sdot_tile16<kNib, false>(g, job0, jobs, njobs, blocks, batch, nullptr, s)
                                          : launch_sdot_tile16<kCrumb, false>(g, job0, jobs, njobs, blocks, batch, nullptr, s);
