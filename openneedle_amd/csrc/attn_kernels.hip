@@ -9,8 +9,9 @@
 // head h of kv head kh = h / G,
 //   s = dot(q_h, float(k_i8)) * k_scale * (1/sqrt(HD))   (sequential over d)
 //   p = softmax(s);  out[d] = sum_s (p_s * v_scale_s) * float(v_i8[s][d]).
-// The dot runs over d in the reference's order but with fused multiply-adds
-// (one rounding per term instead of two), and the value sums likewise. The
+// In the vector kernel the dot runs over d in the reference's order but with
+// fused multiply-adds (one rounding per term instead of two), and the value sums
+// likewise; the matrix kernel forms both from exact integer dots. The
 // softmax and the value sum are computed split-context (flash decoding):
 // each block owns a range of cache slots for one (sequence, kv head) and
 // keeps a running max m, a running sum l and unnormalized outputs o; a merge
@@ -25,7 +26,6 @@
 #include "wave.h"
 
 #include <cmath>
-#include <type_traits>
 
 namespace nd {
 
@@ -323,26 +323,30 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
 // heads G times (measured at 16 sequences x 8 kv heads x 4 heads x 4096 ragged
 // slots of 128: 64 us, 1.4 TB/s of cache). Here both products run on
 // v_mfma_i32_16x16x64_i8 (32 deep for rows of 32) straight from the int8
-// codes, so the cache stream bounds it: 26.4 us there with the merge pass, 29.1 us
-// (4.8 TB/s) at 4096 slots for every sequence.
+// codes, so the cache stream bounds it: 26.4 us there with the merge pass, 29.6 us
+// (4.7 TB/s) at 4096 slots for every sequence.
 //
-// Scores. q is split once per block into four 7-bit digits of a 28-bit fixed
-// point number relative to its head's largest |q| (finer than fp32 there), and
-// the 16 rows of operand A are 4 heads x 4 digits. Operand B is 16 slots' K
-// codes. Output register v of lane l is digit v of head l / 16 and slot l % 16:
-// exact integer dots, joined in the lane with two integer shift-adds and one
-// fused multiply-add.
+// Both operands are split without loss: two groups of four signed 8-bit digits
+// hold 60 bits below the head's largest magnitude. What is left of a q below
+// 2^-36 of the largest is multiplied in fp32; weights below 2^-36 get two more
+// groups, and again until nothing is left. (28 bits of q and 27 of a weight
+// lost the small ones: an outlier in q over zero K codes gave errors of 3e-5 at
+// 1e4 times the rest, 4e-3 at 1e6.) The digit dots are exact integers, and
+// joining them takes a few roundings relative to the sum of the terms'
+// magnitudes, where a chain of fp32 products and sums takes one per term.
 //
-// Values. w = p * v_scale is split the same way relative to the largest w of
-// the head's 64 slots, its bytes transposed so that operand A's rows are heads
-// x digits and its depth the 64 slots; operand B is the V codes, whose rows a
+// Scores. q is split once per block; the 16 rows of operand A are 4 heads x 4
+// digits of a group. Operand B is 16 slots' K codes. Output register v of lane l
+// is digit v of head l / 16 and slot l % 16, joined in the lane.
+//
+// Values. w = p * v_scale is split relative to the largest w of the head's 64
+// slots, its bytes transposed so that operand A's rows are heads x digits and
+// its depth the 64 slots; operand B is the V codes, whose rows a
 // lane loads HD / 16 consecutive bytes at a time (lane l: d = HD / 16 *
 // (l % 16) ..) for 16 slots and transposes with byte permutes (depth byte
 // 4 u + t of lane group l / 16 is slot 16 t + 4 (l / 16) + u). Output register v
 // of lane l is digit v of head l / 16, output d = HD / 16 * (l % 16) + i.
-//
-// The splits keep 27 (q) and 26 (w) bits below the largest term, so the result
-// is at least as close to the exact value as fp32 products and sums.
+// Infinite and NaN weights are multiplied and added slot by slot.
 template <int HD>
 struct MfmaShape {
     static constexpr int kVB = HD / 16;               // V bytes per lane and slot
@@ -363,10 +367,35 @@ __device__ __forceinline__ i32x4 mfma_rows(const i32x4 &a, const i32x4 &b, const
         return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
-// D0 2^21 + D1 2^14 + D2 2^7 + D3 of integer digit sums |D| < 2^21.
+// Two groups of four digits: x below 2^fe is f1 2^(fe - kFirst) + f2 2^(fe - kSecond) + rest, |f1|, |f2| <= 2^30.
+constexpr int kFirst = 30, kSecond = 60;
+
+// The four digits (-128 .. 127, base 256, the lowest first) of f in a dword's bytes.
+__device__ __forceinline__ uint32_t digit_bytes(float f) {
+    // 128 added to every digit, so that no byte borrows from the next, and taken off each byte again
+    return (static_cast<uint32_t>(static_cast<int>(f)) + 0x80808080u) ^ 0x80808080u;
+}
+
+// Both groups of x, which keeps the rest. Exact: what a group leaves is at most
+// half its unit and has x's own last bit, so it fits fp32, and so does f 2^n (f
+// has 24 bits at most from its first to its last).
+__device__ __forceinline__ void take_digits(float &x, int fe, uint32_t &y1, uint32_t &y2) {
+    const float f1 = rintf(ldexpf(x, kFirst - fe));
+    x -= ldexpf(f1, fe - kFirst);
+    const float f2 = rintf(ldexpf(x, kSecond - fe));
+    x -= ldexpf(f2, fe - kSecond);
+    y1 = digit_bytes(f1);
+    y2 = digit_bytes(f2);
+}
+
+// D0 + D1 2^8 + D2 2^16 + D3 2^24 of integer digit sums |D| <= 2^21.
 __device__ __forceinline__ float join_digits(const i32x4 &d) {
-    const int hi = d.x * 128 + d.y, lo = d.z * 128 + d.w;
-    return __builtin_fmaf(static_cast<float>(hi), 16384.0f, static_cast<float>(lo));
+    const int hi = d.w * 256 + d.z, lo = d.y * 256 + d.x;
+    return __builtin_fmaf(static_cast<float>(hi), 65536.0f, static_cast<float>(lo));
+}
+// The two groups' digit sums, in units of the first group's last digit.
+__device__ __forceinline__ float join_groups(const i32x4 &d1, const i32x4 &d2) {
+    return __builtin_fmaf(join_digits(d2), 1.0f / (1 << (kSecond - kFirst)), join_digits(d1));
 }
 
 // 4 x 4 byte transpose: out[i] = byte i of in[0], in[1], in[2], in[3].
@@ -381,22 +410,14 @@ __device__ __forceinline__ void transpose4(const uint32_t (&in)[4], uint32_t (&o
     out[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
 }
 
-// The largest of v over the 16 lanes l % 16 (floats, or absolute bit patterns).
-__device__ __forceinline__ uint32_t row_max(uint32_t v, int lane) {
-    auto step = [&](auto h) {
-        const uint32_t o =
-            __builtin_bit_cast(uint32_t, butterfly_partner<decltype(h)::value>(__builtin_bit_cast(float, v), lane));
-        v = v > o ? v : o;
-    };
-    step(std::integral_constant<int, 1>{});
-    step(std::integral_constant<int, 2>{});
-    step(std::integral_constant<int, 4>{});
-    step(std::integral_constant<int, 8>{});
-    return v;
+// The larger of v and the butterfly partner's (lane ^ H).
+template <int H>
+__device__ __forceinline__ uint32_t max_with(uint32_t v, int lane) {
+    const uint32_t o = __builtin_bit_cast(uint32_t, butterfly_partner<H>(__builtin_bit_cast(float, v), lane));
+    return v > o ? v : o;
 }
 
 constexpr uint32_t kInfBits = 0x7F800000u;
-constexpr int kDigitBias = 64 * (1 + (1 << 7) + (1 << 14) + (1 << 21));
 
 // Block and waves as attn_kernel; sub-tiles of 64 slots as four groups t of 16.
 // Loads of slots not attended read zero (offsets past the buffer).
@@ -407,9 +428,10 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
     constexpr int HQ = (G + 3) / 4;        // quads of heads
     constexpr int GQ = G < 4 ? G : 4;      // heads of a quad
     constexpr uint32_t kOut = 0x80000000u;  // past every buffer (capacity * HD < 2^31)
-    // A operand rows of the value product, 16 bytes of row m = 4 head + digit per 16 slots; a head's four rows
-    // are 80 words apart (the writes of the four heads fall in different banks)
-    __shared__ __attribute__((aligned(16))) uint32_t wd[4][HQ][4 * 80];
+    // A operand rows, 16 bytes of row m = 4 head + digit per lane group; a head's four rows are 80 words apart (the
+    // writes of the four heads fall in different banks)
+    __shared__ __attribute__((aligned(16))) uint32_t wd[4][HQ][2][4 * 80];
+    __shared__ __attribute__((aligned(16))) float qrest[4][HQ][GQ][HD];  // what two groups leave of q (each wave its own copy)
     __shared__ float lred[4][1][G][HD];
     __shared__ float lm[4][G], ll[4][G];
 
@@ -500,48 +522,106 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
     load(cur, st);
     if (store_here && !store_early) store_new<HD>(a, ns, seq, kh, row0);
 
-    // q as operand A: lane (row 4 g + digit, 16-byte chunk quad); qscale: of score lane's head
-    i32x4 q8[HQ][KH];
+    // LDS operations of one wave complete in order; the fences only stop the compiler from moving reads of wd above
+    // the writes before them (and later writes above the reads)
+    auto lds_fence = [] {
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // The lane's operand A of group g from wd: row col = 4 head + digit, lane group quad.
+    auto digits = [&](int hq, int g) {
+        return *reinterpret_cast<const i32x4 *>(wd[wave][hq][g] + (col >> 2) * 80 + (col & 3) * 16 + quad * 4);
+    };
+
+    // q as operand A. Lane (head qg, four-value part qj, chunk quad) splits its four values of each chunk.
+    const int qg = col >> 2, qj = col & 3;
+    const bool qlive = qg < GQ && 4 * qj < KB;
+    i32x4 q8[HQ][2][KH];
+    int qe[HQ];      // of score lane's head: exponent of the first group's last digit
+    bool qleft[HQ];  // wave-uniform: qrest is not all zero
     float qscale[HQ];
 #pragma unroll
     for (int hq = 0; hq < HQ; ++hq) {
-        const int g = col >> 2, digit = col & 3;
-        const bool live = g < GQ;
-        const float *src = qh + (hq * 4 + (live ? g : 0)) * HD + quad * (KB * KH);
-        float x[KH][KB];
+        const int d0 = quad * (KB * KH) + 4 * qj;
+        float x[KH][4];
         uint32_t top = 0;
 #pragma unroll
         for (int h = 0; h < KH; ++h)
 #pragma unroll
-            for (int e = 0; e < KB; ++e) {
-                x[h][e] = live ? src[h * KB + e] : 0.0f;
+            for (int e = 0; e < 4; ++e) {
+                x[h][e] = qlive ? qh[(hq * 4 + qg) * HD + d0 + h * KB + e] : 0.0f;
                 const uint32_t bits = __builtin_bit_cast(uint32_t, x[h][e]) & 0x7FFFFFFFu;
                 top = top > bits ? top : bits;
             }
-        // over the row's four lanes
-        const uint32_t o16 = __builtin_bit_cast(uint32_t, butterfly_partner<16>(__builtin_bit_cast(float, top), lane));
-        top = top > o16 ? top : o16;
-        const uint32_t o32 = __builtin_bit_cast(uint32_t, butterfly_partner<32>(__builtin_bit_cast(float, top), lane));
-        top = top > o32 ? top : o32;
-        const int fe = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, top));  // |q| < 2^fe
+        // over the head's sixteen lanes
+        top = max_with<1>(top, lane);
+        top = max_with<2>(top, lane);
+        top = max_with<16>(top, lane);
+        top = max_with<32>(top, lane);
+        // an infinity or NaN in q makes the head's scores NaN, as its products would
+        const bool finite = top < kInfBits;
+        const int fe = finite ? __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, top)) : 0;  // |q| < 2^fe
+        qscale[hq] = __shfl(finite ? a.scale : __builtin_nanf(""), 4 * quad);
+        qe[hq] = __shfl(fe, 4 * quad) - kFirst;
+        bool left = false;
 #pragma unroll
         for (int h = 0; h < KH; ++h) {
-            uint32_t w[4] = {0, 0, 0, 0};
+            uint32_t y1[4], y2[4], z1[4], z2[4];
 #pragma unroll
-            for (int e = 0; e < KB; ++e) {
-                // bias: 64 in every digit, so that the digits are unsigned and every byte (digit - 64) signed
-                const int y = __float2int_rn(ldexpf(x[h][e], 27 - fe)) + kDigitBias;
-                const int dg = digit == 0 ? y >> 21 : (y >> (7 * (3 - digit))) & 127;
-                w[e >> 2] |= (static_cast<uint32_t>(dg - 64) & 0xFFu) << (8 * (e & 3));
+            for (int e = 0; e < 4; ++e) {
+                x[h][e] = finite ? x[h][e] : 0.0f;
+                take_digits(x[h][e], fe, y1[e], y2[e]);
+                left |= x[h][e] != 0.0f;
             }
-            q8[hq][h] = i32x4{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
+            transpose4(y1, z1);  // z[digit]: the four values' bytes
+            transpose4(y2, z2);
+            const int at = qg * 80 + quad * 4 + qj;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                wd[wave][hq][0][at + i * 16] = z1[i];
+                wd[wave][hq][1][at + i * 16] = z2[i];
+            }
+            lds_fence();
+            q8[hq][0][h] = digits(hq, 0);
+            q8[hq][1][h] = digits(hq, 1);
+            lds_fence();
         }
-        // an infinity or NaN in q makes the head's scores NaN, as its products would
-        const float sc = top >= kInfBits ? __builtin_nanf("") : ldexpf(1.0f, fe - 27);
-        qscale[hq] = __shfl(sc, 4 * quad);
+        qleft[hq] = __any(left);
+        if (qleft[hq] && qlive) {
+#pragma unroll
+            for (int h = 0; h < KH; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) qrest[wave][hq][qg][d0 + h * KB + e] = x[h][e];
+        }
     }
+    lds_fence();
 
-    auto compute = [&](const Tile &T) {
+    // Dots of q's two groups with one slot of the tile, in units of the first group's last digit.
+    auto score = [&](int hq, const i32x4 (&k)[KH]) {
+        i32x4 d1 = {0, 0, 0, 0}, d2 = {0, 0, 0, 0};
+#pragma unroll
+        for (int h = 0; h < KH; ++h) {
+            d1 = mfma_rows<HD>(q8[hq][0][h], k[h], d1);
+            d2 = mfma_rows<HD>(q8[hq][1][h], k[h], d2);
+        }
+        return join_groups(d1, d2);
+    };
+    // The dot of qrest with list position s's K row (read again).
+    auto rest_score = [&](int hq, int s) {
+        const int slot = slot_of(s);
+        const uint32_t kb = slot >= 0 ? static_cast<uint32_t>(slot) * HD : kOut;
+        const float *r = qrest[wave][hq][quad < GQ ? quad : 0];
+        float x = 0.0f;
+#pragma unroll 1
+        for (int d = 0; d < HD; d += 4) {
+            const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(rk, kb + d, 0, 0);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x = __builtin_fmaf(r[d + c], i8f(w, c), x);
+        }
+        return x;
+    };
+
+    auto compute = [&](const Tile &T, int st) {
         // V codes as operand B: depth byte 4 u + t
         i32x4 vt[VB];
 #pragma unroll
@@ -560,12 +640,15 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
             float x[4];
             float top = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                i32x4 d = {0, 0, 0, 0};
+            for (int i = 0; i < 4; ++i) x[i] = ldexpf(score(hq, T.k[i]), qe[hq]);
+            if (qleft[hq]) {
 #pragma unroll
-                for (int h = 0; h < KH; ++h) d = mfma_rows<HD>(q8[hq][h], T.k[i][h], d);
-                x[i] = join_digits(d) * qscale[hq] * T.ks[i];
-                x[i] *= a.scale;
+                for (int i = 0; i < 4; ++i) x[i] += rest_score(hq, st + 16 * i + col);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[i] *= T.ks[i];
+                x[i] *= qscale[hq];
                 x[i] = T.valid[i] ? x[i] : -INFINITY;
                 top = fmaxf(top, x[i]);
             }
@@ -573,52 +656,78 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
             const float alpha = mn == -INFINITY ? 1.0f : expf(m[hq] - mn);
             m[hq] = mn;
             float w[4];
-            uint32_t wtop = 0;
             float ls = 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float e = T.valid[i] ? expf(x[i] - mn) : 0.0f;
                 ls += e;
                 w[i] = e * T.vs[i];
-                const uint32_t bits = __builtin_bit_cast(uint32_t, w[i]) & 0x7FFFFFFFu;
-                wtop = wtop > bits ? wtop : bits;
             }
             l[hq] = l[hq] * alpha + ls;
-            wtop = row_max(wtop, lane);
-            const int fe = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, wtop));  // |w| < 2^fe
-            uint32_t y[4], z[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // 27 bits, biased by 64 in every digit; then 64 off every byte (|f| < 2^26: bytes stay below 128)
-                const uint32_t f = static_cast<uint32_t>(__float2int_rn(ldexpf(w[i], 26 - fe)) + kDigitBias);
-                y[i] = (f >> 21) | (f >> 6 & 0x7F00u) | (f << 9 & 0x7F0000u) | (f << 24 & 0x7F000000u);
-                y[i] = ((y[i] | 0x80808080u) - 0x40404040u) ^ 0x80808080u;
+            for (int i = 0; i < VB; ++i) acc[hq][i] *= alpha;
+            // the lane's largest magnitude, as bits
+            auto top_bits = [&] {
+                uint32_t b = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, w[i]) & 0x7FFFFFFFu;
+                    b = b > bits ? b : bits;
+                }
+                return b;
+            };
+            uint32_t wtop = top_bits();
+            if (__any(wtop >= kInfBits)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+#pragma unroll 1
+                    for (int c = 0; c < 16; ++c) {
+                        const float ww = __shfl(w[i], quad * 16 + c);
+                        if (__builtin_fabsf(ww) < INFINITY) continue;
+                        const uint32_t vb = static_cast<uint32_t>(slot_of(st + 16 * i + c)) * HD + col * VB;
+#pragma unroll
+                        for (int b = 0; b < VB; ++b)
+                            acc[hq][b] += ww * i8f(__builtin_amdgcn_raw_buffer_load_b8(rv, vb + b, 0, 0), 0);
+                    }
+                    w[i] = __builtin_fabsf(w[i]) < INFINITY ? w[i] : 0.0f;
+                }
+                wtop = top_bits();
             }
-            transpose4(y, z);  // z[digit]: bytes t = 0 .. 3
-            uint32_t *dst = wd[wave][hq] + quad * 80 + col;
+            do {
+                wtop = max_with<1>(wtop, lane);
+                wtop = max_with<2>(wtop, lane);
+                wtop = max_with<4>(wtop, lane);
+                wtop = max_with<8>(wtop, lane);
+                const int fe = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, wtop));  // |w| < 2^fe
+                uint32_t y1[4], y2[4], z1[4], z2[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dst[i * 16] = z[i];
-            // LDS operations of one wave complete in order; the fences only stop the compiler from moving the read
-            // above the writes (and the next writes above the read)
-            __builtin_amdgcn_wave_barrier();
-            asm volatile("" ::: "memory");
-            const i32x4 w8 = *reinterpret_cast<const i32x4 *>(wd[wave][hq] + (col >> 2) * 80 + (col & 3) * 16 + quad * 4);
-            __builtin_amdgcn_wave_barrier();
-            asm volatile("" ::: "memory");
-            // an infinite or NaN weight makes the head's outputs NaN
-            const float ws = wtop >= kInfBits ? __builtin_nanf("") : ldexpf(1.0f, fe - 26);
+                for (int i = 0; i < 4; ++i) take_digits(w[i], fe, y1[i], y2[i]);
+                transpose4(y1, z1);  // z[digit]: bytes t = 0 .. 3
+                transpose4(y2, z2);
+                const int at = quad * 80 + col;
 #pragma unroll
-            for (int i = 0; i < VB; ++i) {
-                const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(w8, vt[i], i32x4{0, 0, 0, 0}, 0, 0, 0);
-                acc[hq][i] = __builtin_fmaf(join_digits(d), ws, acc[hq][i] * alpha);
-            }
+                for (int i = 0; i < 4; ++i) {
+                    wd[wave][hq][0][at + i * 16] = z1[i];
+                    wd[wave][hq][1][at + i * 16] = z2[i];
+                }
+                lds_fence();
+                const i32x4 w1 = digits(hq, 0), w2 = digits(hq, 1);
+                lds_fence();
+                wtop = top_bits();
+#pragma unroll
+                for (int i = 0; i < VB; ++i) {
+                    const i32x4 d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, vt[i], i32x4{0, 0, 0, 0}, 0, 0, 0);
+                    const i32x4 d2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2, vt[i], i32x4{0, 0, 0, 0}, 0, 0, 0);
+                    acc[hq][i] += ldexpf(join_groups(d1, d2), fe - kFirst);
+                }
+            } while (__any(wtop != 0));
         }
     };
 
     for (; st < end; st += 256) {
         load(nxt, st + 256);
         asm volatile("" ::: "memory");  // keep the prefetch ahead of the compute
-        compute(cur);
+        compute(cur, st);
         cur = nxt;
     }
 #pragma unroll
@@ -689,8 +798,9 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(const float *__restrict
 
 // One query head per kv head leaves three quarters of the matrix kernel's score
 // lanes idle: at rows of 64 the vector kernel is ahead (64 sequences x 8 kv heads
-// x 2048 slots 24.4 against 24.9 us, one sequence 7.7 against 8.3), at rows of
-// 128 the matrix kernel (8 x 8 x up to 8192 slots 24.4 against 28.0 us).
+// x 2048 slots 24.4 us; the matrix kernel's two heads take 26.2), at rows of 128
+// the matrix kernel in large batches (512 pairs x 600 / 2048 slots 19.0 / 44.8
+// against 20.7 / 46.1 us), and its dots of 128 are closer to the exact value.
 template <int HD, bool SLOTS>
 void launch_attn_hd(const AttnArgs &a, int G, dim3 grid, hipStream_t s) {
     switch (G) {

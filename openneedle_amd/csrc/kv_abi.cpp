@@ -46,10 +46,10 @@ static void check_layer(const KvHandle &kv, int layer) {
 // (sequence, kv head) pairs already (a large decode batch) there is one split
 // and no merge pass, nor on the matrix kernel (whose sums are short enough for
 // it: its error is below the vector kernel's over any number of splits) where
-// the other tiles of a range cost a block less than the merge pass (about 2.5 us: 4 x 8 kv heads x 300 slots of 128, 2
-// heads each, 10.2 -> 8.0 us with one split, 7 x 4 x 777 slots of 32 8.0 ->
-// 6.8 us). A block alone walks a tile in 0.3 us + 2.7 us per 1024 head
-// values (one kv head x 8 heads x 8192 slots of 128: 97 us in one split).
+// the other tiles of a range cost a block less than splitting and merging (4 us).
+// A block alone takes 1.4, 1.6, 2.0 us a tile of 32, 64, 128 values and 1 us more
+// for eight heads: 2 heads of 128, 300 slots 12.1 -> 8.5 us with one split, 128
+// pairs x 600 slots 13.7 -> 11.7; four tiles (1000 slots) 11.2 split, 12.9 not.
 static int auto_splits(int pairs, int length, int group, int head_dim) {
     static const int cus = [] {  // queried once
         int dev = 0, n = 256;
@@ -57,8 +57,8 @@ static int auto_splits(int pairs, int length, int group, int head_dim) {
         return n;
     }();
     const int tiles = (length + 255) / 256;
-    const bool matrix = group > 1 || head_dim == 128;
-    if (matrix && (tiles - 1) * (0.3 + 2.7 * group * head_dim / 1024) < 2.5) return 1;
+    const double tile_us = 1.2 + head_dim / 160.0 + (group > 4 ? 1.0 : 0.0);
+    if ((group > 1 || head_dim == 128) && (tiles - 1) * tile_us < 4.1) return 1;
     const int want = (2 * cus + pairs - 1) / pairs;
     return std::max(1, std::min(want, tiles));
 }
