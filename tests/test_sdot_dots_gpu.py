@@ -56,3 +56,16 @@ def test_int32_accumulators_ragged(bits, group, batch, tile16, monkeypatch):
     x = activations((batch, 1000), seed=batch + 3)
     x[0] = 0
     np.testing.assert_array_equal(device_dots(q, x), oracle_dots(packed, dense.shape, bits, group, cb, x))
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("width,batch", [(8192, 16), (16384, 8), (32768, 4), (8128, 16)])
+def test_widths_that_fill_the_lds(bits, width, batch, monkeypatch):
+    """Groups of 16 at the widths whose activation tile and scales take the quad kernel's whole LDS (the last but one
+    group of them leaves room for the padded rows): the dots, and the outputs on the quad kernel."""
+    monkeypatch.setenv("NEEDLE2_GPU_INT8_QUAD", "always")
+    packed, norms, cb, dense = example(bits, rows=70, dim=width, group=16, seed=width + bits)
+    q = CQMatrix(packed, norms, dense.shape, bits, 16, cb)
+    x = activations((batch, width), seed=batch)
+    np.testing.assert_array_equal(device_dots(q, x), oracle_dots(packed, dense.shape, bits, 16, cb, x))
+    np.testing.assert_array_equal(q.matvec_int8(x), oracle.sdot_linear(packed, norms, dense.shape, bits, 16, cb, x))
