@@ -14,6 +14,12 @@
  *  - int entry points return 0 on success and -1 on failure.
  *  - Calls on one handle must be serialized (needle2/native.py:313);
  *    different handles may be used concurrently (each owns a HIP stream).
+ *  - Calls that take a stream return before the device is done. Device work of
+ *    one handle must not overlap on different streams either where it uses the
+ *    handle's scratch: int8 products and dots, the prefill GEMM, candidates,
+ *    and FP32 products of groups up to 64 wider than 512 inputs or of groups
+ *    above 256. (FP32 products of groups of 128 and 256, and of groups up to 64
+ *    of at most 512 inputs, use none on a caller's stream.)
  */
 #ifndef NEEDLE2_NATIVE_H
 #define NEEDLE2_NATIVE_H

@@ -183,10 +183,14 @@ void CqHandle::gemv(const uint4 *codes, const uint16_t *norms, int rows, int n_p
     matrix_gemv(m, st, codes, norms, rows, n_pad, d_x, d_y, batch, s);
 }
 
+// On the handle's stream its calls follow one another, so st.rot is free for
+// each. On a caller's stream, whose work may overlap that of another call of
+// the handle and may be captured, groups of 128 and 256 take the kernels that
+// transform x themselves.
 void matrix_gemv(const Matrix &m, Staging &st, const uint4 *codes, const uint16_t *norms, int rows, int n_pad,
                  const float *d_x, float *d_y, int batch, hipStream_t s) {
     const float *act = d_x;
-    const GemvPath path = gemv_path(m.kind, m.group, m.in, m.dev, n_pad / kRowsPerBlock, batch);
+    const GemvPath path = gemv_path(m.kind, m.group, m.in, m.dev, n_pad / kRowsPerBlock, batch, st.owns(s));
     if (!path.raw) {
         st.rot.reserve(size_t(batch) * m.dev);
         if (gemv_prepass(m.group))

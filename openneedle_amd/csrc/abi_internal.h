@@ -65,6 +65,7 @@ struct Matrix {
 // device-resident callers pass their own) and grow-only staging buffers.
 struct Staging {
     hipStream_t stream();
+    bool owns(hipStream_t s) const { return stream_ && s == stream_; }
     DevBuf<float> x, rot, y, big, xs, xst;
     DevBuf<int32_t> q;
     DevBuf<_Float16> xh;  // fp16 transformed activations of the prefill GEMM

@@ -262,7 +262,9 @@ void launch_rot_many(const float *x0, const float *const *xptr, int batch, int n
 struct GemvPath {
     bool batched, raw;
 };
-GemvPath gemv_path(int kind, int group, int in, int dev, int blocks, int batch);
+// scratch: the caller has a buffer for transformed rows that nothing else uses meanwhile; without one, groups of 128
+// and 256 take the kernels that transform the raw input (other groups' callers bring one where the path needs it).
+GemvPath gemv_path(int kind, int group, int in, int dev, int blocks, int batch, bool scratch = true);
 // njobs == 0: one job passed by value (job0); otherwise jobs_dev[0..njobs). The batch kernel takes every job's rows
 // from `batch`, the one-row kernels from the jobs.
 void launch_cq_gemv(const CqGeom &g, const CqJob &job0, const CqJob *jobs_dev, int njobs, int total_blocks, int batch,

@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from openneedle_amd.cq import CQMatrix, Plan
-from openneedle_amd.device import DeviceArray, synchronize
+from openneedle_amd.device import DeviceArray, Graph, Stream, synchronize
 from tests.cases import activations, example
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +61,42 @@ def test_batch_special_values():
     q = CQMatrix(packed, norms, dense.shape, 4, 64, cb)
     got = q.matvec(x)
     np.testing.assert_array_equal(got, expected)
+
+
+@pytest.mark.parametrize("bits,group", [(4, 128), (2, 256)])
+def test_one_handle_on_two_streams(bits, group):
+    """Groups of 128 and 256 use no scratch of the handle on a caller's stream: products of different inputs enqueued on
+    two streams, whose work may overlap, do not disturb each other, and neither does one on the handle's own."""
+    packed, norms, cb, dense = example(bits, rows=3000, dim=4000, group=group, seed=group)
+    q = CQMatrix(packed, norms, dense.shape, bits, group, cb)
+    xs = [activations((4, 4000), seed=k) for k in range(3)]
+    want = [oracle.cq_linear(packed, norms, dense.shape, bits, group, cb, x, 8) for x in xs]
+    streams = [Stream(), Stream(), None]  # None: the handle's stream
+    d_x = [DeviceArray.from_host(x) for x in xs]
+    d_y = [[DeviceArray(want[0].nbytes) for _ in range(20)] for _ in streams]
+    for n in range(20):
+        for k, s in enumerate(streams):
+            q.matvec_device(d_x[k].ptr, d_y[k][n].ptr, 4, s)
+    synchronize()
+    for k, w in enumerate(want):
+        for y in d_y[k]:
+            np.testing.assert_array_equal(y.to_host(np.float32, w.shape), w)
+
+
+@pytest.mark.parametrize("group", [128, 256])
+def test_first_call_in_a_capture(group):
+    """A handle's first product may be captured: nothing is allocated for groups of 128 and 256."""
+    packed, norms, cb, dense = example(4, rows=300, dim=1100, group=group, seed=group)
+    warm, q = [CQMatrix(packed, norms, dense.shape, 4, group, cb) for _ in range(2)]
+    x = activations((4, 1100), seed=8)
+    want = oracle.cq_linear(packed, norms, dense.shape, 4, group, cb, x, 4)
+    d_x, d_y, s = DeviceArray.from_host(np.zeros_like(x)), DeviceArray(want.nbytes), Stream()
+    warm.matvec_device(d_x.ptr, d_y.ptr, 4, s)  # loads the kernel
+    s.synchronize()
+    with Graph.capture(s) as graph:
+        q.matvec_device(d_x.ptr, d_y.ptr, 4, s)
+    for scale in (1, 2, 4):
+        d_x.upload(x * np.float32(scale))
+        graph.launch(s)
+        s.synchronize()
+        np.testing.assert_array_equal(d_y.to_host(np.float32, want.shape), want * np.float32(scale))
