@@ -6,6 +6,11 @@ the 1e-5 relative / 1e-6 absolute per-output requirement. Results are also
 checked against the fp64 dense closed form with the reference test's
 tolerance (atol=3e-6, rtol=2e-5, tests/test_native.py:40 in the reference).
 """
+import os
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -240,3 +245,31 @@ def test_linear_many_falls_back_per_matrix():
     x = activations(512, seed=951)
     for out, ref in zip(matvec_many(mats, x), refs):
         np.testing.assert_array_equal(out, oracle.cq_linear(*ref, x))
+
+
+LONG_CALL = """
+import ctypes, time
+from openneedle_amd import _ffi
+_ffi.lib()
+assert ctypes.CDLL("libamdhip64.so").hipSetDeviceFlags(4) == 0  # hipDeviceScheduleBlockingSync
+from openneedle_amd.cq import CQMatrix
+from tests.cases import activations, baseline
+packed, norms, cb, _ = baseline(4, 4096, 8192)
+q, x = CQMatrix(packed, norms, (4096, 8192), 4, 32, cb), activations((256, 8192))
+q.matvec(x)
+wall, cpu = time.perf_counter(), time.thread_time()
+for _ in range(5):
+    q.matvec(x)
+print("long call:", time.thread_time() - cpu, time.perf_counter() - wall)
+"""
+
+
+def test_long_host_call_sleeps_under_blocking_sync():
+    """A host-pointer product of milliseconds (one row per pass over the codes) leaves the core to others where the
+    program chose blocking waits: most of its time is not the calling thread's."""
+    env = dict(os.environ, NEEDLE2_GPU_FP32_PAIRS="never")
+    out = subprocess.run([sys.executable, "-c", LONG_CALL], env=env, cwd=Path(__file__).resolve().parents[1], timeout=100,
+                         capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    cpu, wall = (float(v) for v in out.stdout.split("long call:")[1].split())
+    assert cpu < wall / 2, (cpu, wall)
