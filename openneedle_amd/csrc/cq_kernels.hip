@@ -1481,11 +1481,12 @@ static bool gemv_quad_takes_x(int group, int in) {
 // and 32 row tiles or more (8 x 2048 x 4000 g128: 50.9 against 58.6 us; 2048 x
 // 512 11.3 against 8.8), the rest the pair kernel or one row per pass (CQ4 g32
 // 52.0 against 48.8, CQ2 g64 47.8 against 35.8). Its buffer resource spans
-// eight rows, which must stay under 2^32 bytes.
+// eight rows, which must stay under 2^32 bytes, and it and its pre-pass have the
+// batch in the grid's y, which ends at 65535.
 GemvPath gemv_path(int kind, int group, int in, int dev, int blocks, int batch, bool scratch) {
     const bool enough = batch >= 4 || (batch == 3 && !(kind == kCrumb && group <= 64)) ||
                         (batch == 2 && kind == kNib && group > 64 && blocks >= 32);
-    const bool batched = enough && dev <= 1 << 26 && !one_row_forced() && (scratch || !gemv_fuses_fwht(group));
+    const bool batched = enough && batch <= 65535 && dev <= 1 << 26 && !one_row_forced() && (scratch || !gemv_fuses_fwht(group));
     return {batched, gemv_quad_takes_x(group, in) || (gemv_fuses_fwht(group) && !batched)};
 }
 

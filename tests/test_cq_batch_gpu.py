@@ -100,3 +100,12 @@ def test_first_call_in_a_capture(group):
         graph.launch(s)
         s.synchronize()
         np.testing.assert_array_equal(d_y.to_host(np.float32, want.shape), want * np.float32(scale))
+
+
+@pytest.mark.parametrize("group", [32, 128])
+def test_more_rows_than_a_grid_holds(group):
+    """70000 rows: past the 65535 blocks of a grid's y, one row per pass over the codes in one launch."""
+    packed, norms, cb, dense = example(4, rows=3, dim=128, group=group, seed=group)
+    x = activations((70000, 128), seed=1)
+    q = CQMatrix(packed, norms, dense.shape, 4, group, cb)
+    np.testing.assert_array_equal(q.matvec(x), oracle.cq_linear(packed, norms, dense.shape, 4, group, cb, x, 8))
