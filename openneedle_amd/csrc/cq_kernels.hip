@@ -1475,18 +1475,38 @@ static bool gemv_quad_takes_x(int group, int in) {
     return in <= 2 * kWindow;
 }
 
-// The batch kernel from four rows on, and from three except for 2-bit groups
-// of up to 64 (8 x 2048 x 4000: 52.0 against 50.5 us one row per pass; CQ4 g32
-// 57.8 against 72.0 in pairs). Two rows take it only for 4-bit groups above 64
-// and 32 row tiles or more (8 x 2048 x 4000 g128: 50.9 against 58.6 us; 2048 x
-// 512 11.3 against 8.8), the rest the pair kernel or one row per pass (CQ4 g32
-// 52.0 against 48.8, CQ2 g64 47.8 against 35.8). Its buffer resource spans
-// eight rows, which must stay under 2^32 bytes, and it and its pre-pass have the
-// batch in the grid's y, which ends at 65535.
+// Whether the batch kernel pays against one row per pass (two 4-bit rows of
+// groups up to 64: the pair kernel). Groups of 128 and 256 then need the
+// pre-pass that one row per pass does without, some 3 us, so their line lies
+// where the rows' walks cost more: `walk` counts windows walked again after the
+// first row, groups of 256 (whose one-row walk takes twice as long) twice.
+// Plans of 32 and more row tiles, one row per pass against the batch kernel:
+// CQ4 g128, 2 rows, 512 / 1100 / 2048 columns 8.9 / 20.3 / 30.3 against 11.3 /
+// 22.6 / 28.0 us, 3 rows, 256 / 512 8.7 / 12.2 against 10.2 / 11.5; CQ4 g256, 2
+// rows, 768 / 1100 18.8 / 29.4 against 19.5 / 27.7; CQ2 g128, 3 rows, 768 / 1100
+// 15.9 / 24.2 against 18.1 / 23.1, 4 rows, 512 / 768 12.1 / 20.4 against 13.2 /
+// 18.1; CQ2 g256, 3 rows, 512 / 1100 14.2 / 30.4 against 15.5 / 28.0. Other
+// groups, whose rows are transformed ahead either way: from four rows on, and
+// from three except for 2-bit groups of up to 64 (8 x 2048 x 4000: 52.0 against
+// 50.5 us one row per pass; CQ4 g32 57.8 against 72.0 in pairs); two rows only
+// of 4-bit groups above 256 and from 32 row tiles on (CQ4 g32 52.0 against 48.8,
+// CQ2 g64 47.8 against 35.8).
+static bool batch_pays(int kind, int group, int in, int blocks, int batch) {
+    if (gemv_fuses_fwht(group)) {
+        const long walk = static_cast<long>(batch - 1) * ((in + kWindow - 1) / kWindow) * (group / 128);
+        if (kind == kCrumb) return batch >= 6 || (batch >= 3 && walk >= 9);
+        return batch >= 4 || (batch == 3 && walk >= 4) || (batch == 2 && walk >= 8 && blocks >= 32);
+    }
+    return batch >= 4 || (batch == 3 && !(kind == kCrumb && group <= 64)) ||
+           (batch == 2 && kind == kNib && group > 64 && blocks >= 32);
+}
+
+// The batch kernel's buffer resource spans eight rows, which must stay under
+// 2^32 bytes, and it and its pre-pass have the batch in the grid's y, which ends
+// at 65535.
 GemvPath gemv_path(int kind, int group, int in, int dev, int blocks, int batch, bool scratch) {
-    const bool enough = batch >= 4 || (batch == 3 && !(kind == kCrumb && group <= 64)) ||
-                        (batch == 2 && kind == kNib && group > 64 && blocks >= 32);
-    const bool batched = enough && batch <= 65535 && dev <= 1 << 26 && !one_row_forced() && (scratch || !gemv_fuses_fwht(group));
+    const bool batched = batch_pays(kind, group, in, blocks, batch) && batch <= 65535 && dev <= 1 << 26 &&
+                         !one_row_forced() && (scratch || !gemv_fuses_fwht(group));
     return {batched, gemv_quad_takes_x(group, in) || (gemv_fuses_fwht(group) && !batched)};
 }
 
