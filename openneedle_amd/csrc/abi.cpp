@@ -200,7 +200,7 @@ void matrix_gemv(const Matrix &m, Staging &st, const uint4 *codes, const uint16_
             m.transform(d_x, m.in, st.rot.p, batch, st.big, s);
         act = st.rot.p;
     }
-    const CqJob job{codes, norms, act, d_y, rows, n_pad, 0, batch, 0};
+    const CqJob job{codes, norms, act, d_y, rows, 0, batch, 0};
     launch_cq_gemv(m.geom(), job, nullptr, 0, n_pad / kRowsPerBlock, batch, path, s);
 }
 
@@ -497,7 +497,7 @@ static void plan_upload(Plan &p) {
         for (int i = 0; i < p.count; ++i) {
             const Matrix &mi = p.cq[i]->m;
             const float *act = p.path.raw ? p.xs_in[i] : p.rot.p + size_t(i) * p.batch * m.dev;
-            jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, p.ys[i], mi.out, mi.n_pad, block, p.batch, 0};
+            jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, p.ys[i], mi.out, block, p.batch, 0};
             block += mi.n_pad / kRowsPerBlock;
         }
         host.assign(reinterpret_cast<uint8_t *>(jobs.data()), reinterpret_cast<uint8_t *>(jobs.data() + p.count));
@@ -676,7 +676,7 @@ static void linear_many(const std::vector<CqHandle *> &hs, const float *x, float
             runs.push_back({i, 0});
             block = 0;
         }
-        jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, st.y.p + at[i], mi.out, mi.n_pad, block, 1, 0};
+        jobs[i] = CqJob{mi.codes.p, mi.norms.p, act, st.y.p + at[i], mi.out, block, 1, 0};
         block += mi.n_pad / kRowsPerBlock;
         runs.back().second = block;
     }

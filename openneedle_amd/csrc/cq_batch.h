@@ -345,7 +345,6 @@ __global__ __launch_bounds__(kRowsPerBlock *KS, 2) void cq_gemv_batch_kernel(CqJ
         J.act = cj[j].act;
         J.y = cj[j].y;
         J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
         J.block_begin = cj[j].block_begin;
         J.ystride = cj[j].ystride;
     }

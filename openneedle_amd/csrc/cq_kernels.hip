@@ -418,7 +418,6 @@ __global__ __launch_bounds__(kRowsPerBlock, 2) void cq_gemv_kernel(CqJob job0, c
         J.act = cj[j].act;
         J.y = cj[j].y;
         J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
         J.block_begin = cj[j].block_begin;
         J.batch = cj[j].batch;
     }
@@ -752,7 +751,6 @@ __global__ __launch_bounds__(kSplitThreads, 4) void cq_gemv_split_kernel(CqJob j
         J.act = cj[j].act;
         J.y = cj[j].y;
         J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
         J.block_begin = cj[j].block_begin;
         J.batch = cj[j].batch;
     }
@@ -851,7 +849,6 @@ __global__ __launch_bounds__(kWsplitThreads) void cq_gemv_wsplit_kernel(CqJob jo
         J.act = cj[j].act;
         J.y = cj[j].y;
         J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
         J.block_begin = cj[j].block_begin;
         J.batch = cj[j].batch;
     }
@@ -1217,7 +1214,6 @@ __global__ __launch_bounds__(kQuadThreads) __attribute__((amdgpu_waves_per_eu(8,
         J.act = cj[j].act;
         J.y = cj[j].y;
         J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
         J.block_begin = cj[j].block_begin;
         J.batch = cj[j].batch;
     }
@@ -1252,7 +1248,6 @@ __global__ __launch_bounds__(kQuadThreads) __attribute__((amdgpu_waves_per_eu(4,
         J.act = cj[j].act;
         J.y = cj[j].y;
         J.rows = cj[j].rows;
-        J.n_pad = cj[j].n_pad;
         J.block_begin = cj[j].block_begin;
         J.batch = cj[j].batch;
     }

@@ -118,7 +118,7 @@ struct GemvGroup {
                 const float *act = path.raw ? input + size_t(t) * m0->in : rot.p + size_t(t) * m0->dev;
                 host.push_back(CqJob{p.m->codes.p + size_t(tile0) * p.m->chunks * kRowsPerBlock,
                                      p.m->norms.p + size_t(tile0) * p.m->groups * kRowsPerBlock, act,
-                                     p.y + size_t(t) * p.ystride, rows, tiles * kRowsPerBlock, blocks, 1, p.ystride});
+                                     p.y + size_t(t) * p.ystride, rows, blocks, 1, p.ystride});
                 blocks += tiles;
             }
         };
