@@ -1843,15 +1843,17 @@ static bool tile16_wanted(int batch) {
 }
 
 // The fp16 batch kernel (sdot_batch.hip): 4-bit codes in groups of 32 or 64, 2
-// .. 12 rows, or 128, 2 .. 8 rows (NEEDLE2_GPU_INT8_BATCH "always" / "never";
+// .. 12 rows, or 128, 5 .. 8 rows (NEEDLE2_GPU_INT8_BATCH "always" / "never";
 // an override of one of the kernels it stands before leaves it out). 32 x CQ4
 // 4096 x 4096 against the quad kernel (tile16 at 12 rows): g32 at 2 / 4 / 8 /
 // 12 rows 55 / 63 / 77 / 92 against 68 / 73 / 95 / 104 us, g64 52 / 55 / 73 /
-// 90 against 61 / 62 / 80 / 104, g128 53 / 57 / 70 against 54 / 59 / 77. Its
-// table costs each workgroup some 2 us, so it takes 384 row tiles and, under
-// four rows, 8192 windows of them (g128: 24 x 5003 x 3000 at 3 / 5 rows 39.5 /
-// 44.4 against 36.2 / 48.1, 6 x 8000 x 2000 at 2 rows 20.7 against 18.0). At 16
-// rows its 4 x 4 x 4 products take longer than tile16 (116 against 110).
+// 90 against 61 / 62 / 80 / 104, g128 70 against 77 at 8 rows, even at 2 to 4.
+// Up to one row tile per CU the others keep up at few rows: their time over its
+// time at 256 tiles x 4096 columns and 4 / 6 / 12 rows is g32 0.96 / 1.31 / 1.10,
+// g64 0.84 / 0.96 / 1.36, g128 0.81 / 0.95; at 320 tiles 1.08 / 1.36 / 1.28, 0.99 /
+// 1.09 / 1.51, 0.95 / 1.06 (512 to 8192 columns alike). So there it takes groups
+// of 32 from five rows on, and nine rows and more. At 16 rows its 4 x 4 x 4
+// products take longer than tile16 (116 against 110).
 static bool batch_wanted(const SdotGeom &g, int blocks, int batch) {
     const char *mode = std::getenv("NEEDLE2_GPU_INT8_BATCH");
     if (mode && (std::strcmp(mode, "always") == 0 || std::strcmp(mode, "never") == 0)) return mode[0] == 'a';
@@ -1859,8 +1861,9 @@ static bool batch_wanted(const SdotGeom &g, int blocks, int batch) {
         const char *other = std::getenv(name);
         if (other && (std::strcmp(other, "always") == 0 || std::strcmp(other, "never") == 0)) return false;
     }
-    if (blocks < 384 || (batch < 4 && static_cast<long>(blocks) * g.windows < 8192)) return false;
-    return g.group <= 128 && batch <= (g.group <= 64 ? 12 : 8);
+    if (g.group > 128 || batch > (g.group <= 64 ? 12 : 8)) return false;
+    if (blocks <= device_cus()) return batch > 8 || (g.group == 32 && batch > 4);
+    return g.group <= 64 || batch > 4;
 }
 
 // The K split for small matrices (NEEDLE2_GPU_INT8_KSPLIT "always" / "never") and, within it, the 16 x 16
@@ -1920,6 +1923,8 @@ void launch_sdot_gemv(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
     //    on 16 x 16 tiles at batch 2 and more (NEEDLE2_GPU_INT8_KS16:
     //    "never", or "always" from batch 1);
     //  - one batch row: the barrier-free row kernel (NEEDLE2_GPU_INT8_ROW);
+    //  - 2 to 12 rows of 4-bit groups of 32 to 128, by batch_wanted: the fp16
+    //    batch kernel of sdot_batch.hip (NEEDLE2_GPU_INT8_BATCH);
     //  - 9 or more: batch tiles of 16 rows on v_mfma_i32_16x16x32_i8, every
     //    code decoded once per tile (NEEDLE2_GPU_INT8_TILE16);
     //  - 2 or more: batch tiles of up to 16 rows on v_mfma_i32_4x4x4_16b_i8,
