@@ -29,6 +29,16 @@ const char *get_error();
         if (nd_e_ != hipSuccess) nd::hip_fail(#expr, nd_e_, __FILE__, __LINE__); \
     } while (0)
 
+// Compute units of the device (queried once).
+inline int device_cus() {
+    static int cus = [] {
+        int dev = 0, n = 256;
+        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        return n;
+    }();
+    return cus;
+}
+
 // Waits for the stream by polling it instead of hipStreamSynchronize, whose
 // wake-up measured 2-10% of an engine decode step (~650 us of kernels that end
 // by writing pinned host memory); the host thread spins while the stream runs.

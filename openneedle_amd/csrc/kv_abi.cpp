@@ -49,17 +49,13 @@ static void check_layer(const KvHandle &kv, int layer) {
 // the other tiles of a range cost a block less than splitting and merging (4 us).
 // A block alone takes 1.4, 1.6, 2.0 us a tile of 32, 64, 128 values and 1 us more
 // for eight heads: 2 heads of 128, 300 slots 12.1 -> 8.5 us with one split, 128
-// pairs x 600 slots 13.7 -> 11.7; four tiles (1000 slots) 11.2 split, 12.9 not.
+// pairs x 600 slots 13.7 -> 11.3; one head, four tiles (1000 slots) 10.5 split,
+// 12.6 not.
 static int auto_splits(int pairs, int length, int group, int head_dim) {
-    static const int cus = [] {  // queried once
-        int dev = 0, n = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        return n;
-    }();
     const int tiles = (length + 255) / 256;
     const double tile_us = 1.2 + head_dim / 160.0 + (group > 4 ? 1.0 : 0.0);
     if ((group > 1 || head_dim == 128) && (tiles - 1) * tile_us < 4.1) return 1;
-    const int want = (2 * cus + pairs - 1) / pairs;
+    const int want = (2 * device_cus() + pairs - 1) / pairs;
     return std::max(1, std::min(want, tiles));
 }
 

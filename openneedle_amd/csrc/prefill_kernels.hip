@@ -628,14 +628,13 @@ void launch_prefill_transform(const float *x, int m, int in, int padded, int dev
 
 namespace {
 
-// 256-row tiles where they save rounds of the 256 CUs: a tall tile's step takes
+// 256-row tiles where they save rounds of the CUs: a tall tile's step takes
 // 0.91 us against 0.67 (1999 x 11008 x 4096, group 128: three rounds instead of
 // six, 262 -> 196 us with the transform); 512 x 8192 x 2048 fills one round
 // with low tiles and would leave half the CUs idle with tall ones.
 bool tall_tiles(int ntiles, int m) {
-    const int low = (ntiles * ((m + kBM - 1) / kBM) + 255) / 256;
-    const int tall = (ntiles * ((m + 2 * kBM - 1) / (2 * kBM)) + 255) / 256;
-    return tall * 1.4 < low;
+    auto rounds = [&](int bm) { return (ntiles * ((m + bm - 1) / bm) + device_cus() - 1) / device_cus(); };
+    return rounds(2 * kBM) * 1.4 < rounds(kBM);
 }
 
 template <bool TALL>

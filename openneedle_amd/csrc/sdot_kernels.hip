@@ -1599,15 +1599,6 @@ bool launch_sdot_ks16(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
     return true;
 }
 
-int device_cus() {
-    static int cus = [] {
-        int dev = 0, n = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        return n;
-    }();
-    return cus;
-}
-
 // The batch is covered by tiles of 16, 8, 4, 2 and 1 rows (largest first),
 // one tile per blockIdx.y. A tile size that would leave fewer than two
 // workgroups per CU is skipped: small matrices with many batch rows (a
