@@ -817,15 +817,16 @@ constexpr int kQuadMaxLds = 160 * 1024;
 // 99 us. tile16's 16-byte reads of 2-bit matrices measured no faster with it
 // (g128, batch 16: 59 us without). The quad kernel drops it for the widths that
 // fill the LDS without it (groups of 16: 8129 .. 8192 at tiles of 16 rows, 16321
-// .. 16384 at 8, 32705 .. 32768 at 4); no width of tile16 comes that close.
+// .. 16384 at 8, 32705 .. 32768 at 4; no other group's and no tile16 width comes
+// that close), as a kernel of its own: with a row length known only at run time 64
+// x CQ2 701 x 2048 g128 at 6 rows took 21.3 us against 20.0.
 constexpr int kRowPad = 4;
 template <int KIND>
 constexpr int kTile16Pad = KIND == kNib ? kRowPad : 0;
 
-template <int KIND, int GROUP, int NQ, bool DOTS>
+template <int KIND, int GROUP, int NQ, bool DOTS, int PAD = kRowPad>
 __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, const SdotJob *__restrict__ jobs,
-                                                                 int njobs, SdotGeom geom, int32_t *__restrict__ dots,
-                                                                 int pad) {
+                                                                 int njobs, SdotGeom geom, int32_t *__restrict__ dots) {
     using S = RowSlot<KIND, GROUP>;
     constexpr int TB = 4 * NQ;  // batch rows of the tile
     extern __shared__ __attribute__((aligned(16))) uint32_t quad_lds[];
@@ -849,7 +850,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, 
     const int groups = geom.groups;
     const int dev = geom.windows * kWindow;
     const int qdw = dev / 4;  // activation dwords per batch row
-    const int ldw = qdw + pad;  // and in LDS
+    const int ldw = qdw + PAD;  // and in LDS
     const int b0 = static_cast<int>(blockIdx.y) * TB;
     const int nb = min(TB, J.batch - b0);  // valid batch rows of the tile (uniform)
     uint32_t *lq = quad_lds;
@@ -868,7 +869,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void sdot_quad_kernel(SdotJob job0, 
     // stage the tile's activation rows and group scales (rows past the batch as zeros)
     const u32x4 *q4 = reinterpret_cast<const u32x4 *>(J.q) + static_cast<size_t>(b0) * (qdw / 4);
     for (int i = threadIdx.x; i < TB * qdw / 4; i += kRowsPerBlock)
-        reinterpret_cast<u32x4 *>(lq)[i + i / (qdw / 4) * (pad / 4)] =
+        reinterpret_cast<u32x4 *>(lq)[i + i / (qdw / 4) * (PAD / 4)] =
             i / (qdw / 4) < nb ? q4[i] : u32x4{0, 0, 0, 0};
     for (int i = threadIdx.x; i < TB * groups; i += kRowsPerBlock)
         lxs[i] = i / groups < nb ? J.xs[static_cast<size_t>(b0) * groups + i] : 0.0f;
@@ -959,8 +960,8 @@ bool launch_sdot_quad(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
     const int dev = g.windows * kWindow;
     const int tb = batch >= 16 ? 16 : (batch + 3) / 4 * 4;  // rows per tile
     const size_t bare = static_cast<size_t>(tb) * dev + static_cast<size_t>(tb) * g.groups * 4;
-    const int pad = bare + static_cast<size_t>(tb) * 4 * kRowPad <= kQuadMaxLds ? kRowPad : 0;
-    const size_t lds = bare + static_cast<size_t>(tb) * 4 * pad;
+    const bool padded = g.group != 16 || bare + static_cast<size_t>(tb) * 4 * kRowPad <= kQuadMaxLds;
+    const size_t lds = bare + (padded ? static_cast<size_t>(tb) * 4 * kRowPad : 0);
     if (lds > kQuadMaxLds || g.group > kWindow) return false;
     dim3 grid(blocks, (batch + tb - 1) / tb), block(kRowsPerBlock);
     auto go = [&](auto nq) {
@@ -968,15 +969,18 @@ bool launch_sdot_quad(const SdotGeom &g, const SdotJob &job0, const SdotJob *job
         switch (g.group) {
         case 8:
             if constexpr (KIND == kNib) {
-                hipLaunchKernelGGL((sdot_quad_kernel<KIND, 8, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots, pad);
+                hipLaunchKernelGGL((sdot_quad_kernel<KIND, 8, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots);
                 break;
             }
             [[fallthrough]];
-        case 16: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 16, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots, pad); break;
-        case 32: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 32, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots, pad); break;
-        case 64: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 64, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots, pad); break;
-        case 128: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 128, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots, pad); break;
-        default: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 256, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots, pad); break;
+        case 16:
+            if (padded) hipLaunchKernelGGL((sdot_quad_kernel<KIND, 16, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots);
+            else hipLaunchKernelGGL((sdot_quad_kernel<KIND, 16, NQ, DOTS, 0>), grid, block, lds, s, job0, jobs, njobs, g, dots);
+            break;
+        case 32: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 32, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots); break;
+        case 64: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 64, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots); break;
+        case 128: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 128, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots); break;
+        default: hipLaunchKernelGGL((sdot_quad_kernel<KIND, 256, NQ, DOTS>), grid, block, lds, s, job0, jobs, njobs, g, dots); break;
         }
     };
     switch (tb / 4) {
