@@ -32,6 +32,8 @@
 
 #include <hip/hip_fp16.h>
 
+#include <cstdio>
+#include <cstdlib>
 #include <type_traits>
 #include <utility>
 
@@ -378,15 +380,26 @@ struct BatchPick {
 // its MFMAs and ~2 for the centroid lookups; below two waves per SIMD it runs
 // 1.6 times slower (27.7 against 17.4 ns, see above). Fewer rows per tile
 // repeat the lookups, more rows leave SIMDs idle; four parts divide a row's
-// walk by four where tiles alone do not fill the chip.
+// walk by four where tiles alone do not fill the chip. NEEDLE2_GPU_FP32_BATCH =
+// "rows,parts" picks them, where the group has such a kernel.
 BatchPick pick(const CqGeom &g, int blocks, int batch) {
     constexpr int kSimds = 1024;
+    auto parts_ok = [&](int ks) {
+        return ks == 1 || (g.group >= 32 && g.groups * (g.group < 64 ? g.group : 64) >= 4 * 64 && g.groups >= 4);
+    };
+    auto rows_ok = [&](int nb) { return g.group >= 32 || (nb != 3 && nb != 6); };
+    if (const char *mode = std::getenv("NEEDLE2_GPU_FP32_BATCH")) {
+        int nb = 0, ks = 0;
+        if (std::sscanf(mode, "%d,%d", &nb, &ks) == 2 && (ks == 1 || ks == 4) && parts_ok(ks) &&
+            (nb == 2 || nb == 3 || nb == 4 || nb == 6 || nb == 8) && rows_ok(nb))
+            return {nb, ks};
+    }
     BatchPick best{2, 1};
     double cost = 0;
     for (int ks : {1, 4}) {
-        if (ks > 1 && (g.group < 32 || g.groups * (g.group < 64 ? g.group : 64) < 4 * 64 || g.groups < 4)) continue;
+        if (!parts_ok(ks)) continue;
         for (int nb : {2, 3, 4, 6, 8}) {
-            if (g.group < 32 && (nb == 3 || nb == 6)) continue;
+            if (!rows_ok(nb)) continue;
             const double waves = 4.0 * ks * blocks * ((batch + nb - 1) / nb);
             const double per_simd = waves / kSimds;
             const double turns = per_simd <= 1 ? 1.6 : per_simd <= 2 ? 2 : per_simd;

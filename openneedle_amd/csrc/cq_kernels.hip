@@ -1277,7 +1277,8 @@ __global__ __launch_bounds__(kRowsPerBlock) void rot_many_kernel(const float *__
     if (p < dev) rot[static_cast<size_t>(v) * dev + p] = x[0];
 }
 
-// NEEDLE2_GPU_FP32_PAIRS=never: batches run one row per pass over the codes.
+// NEEDLE2_GPU_FP32_PAIRS=never: batches run one row per pass over the codes, on neither the pair nor the batch
+// kernel (an engine's long prompt chunks stay on the batch kernel).
 static bool one_row_forced() {
     const char *mode = std::getenv("NEEDLE2_GPU_FP32_PAIRS");
     return mode && std::strcmp(mode, "never") == 0;
@@ -1486,7 +1487,9 @@ static bool gemv_quad_takes_x(int group, int in) {
 // 50.5 us one row per pass; CQ4 g32 57.8 against 72.0 in pairs); two rows only
 // of 4-bit groups above 256 and from 32 row tiles on (CQ4 g32 52.0 against 48.8,
 // CQ2 g64 47.8 against 35.8).
+// NEEDLE2_GPU_FP32_BATCH, the kernel's own override (cq_batch.h), takes every batch of two and more.
 static bool batch_pays(int kind, int group, int in, int blocks, int batch) {
+    if (std::getenv("NEEDLE2_GPU_FP32_BATCH")) return batch >= 2;
     if (gemv_fuses_fwht(group)) {
         const long walk = static_cast<long>(batch - 1) * ((in + kWindow - 1) / kWindow) * (group / 128);
         if (kind == kCrumb) return batch >= 6 || (batch >= 3 && walk >= 9);

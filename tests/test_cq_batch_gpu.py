@@ -1,8 +1,8 @@
 """The FP32 batch GEMV (cq_batch.h): several activation rows per pass over the codes, products on the matrix cores.
 
-Bit-identical to the oracle at every tile height (2, 3, 4, 6, 8 rows, a last tile of fewer), for groups below, equal
-to and above one block of 64 positions, with the K walk in one part and in four (rows of at least four groups and
-256 positions), odd widths and rows, raw (up to 512 wide) and transformed inputs.
+Bit-identical to the oracle at every tile height (2, 3, 4, 6, 8 rows, a last tile of fewer) with the K walk in one part
+and in four (forced: test_every_tile_and_part), and in the launches that sizes pick, for groups below, equal to and
+above one block of 64 positions, odd widths and rows, raw (up to 512 wide) and transformed inputs.
 """
 import numpy as np
 import pytest
@@ -13,6 +13,32 @@ from openneedle_amd.device import DeviceArray, Graph, Stream, synchronize
 from tests.cases import activations, example
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("group", [8, 16, 32, 64, 128, 256, 512])
+@pytest.mark.parametrize("nb,parts", [(nb, ks) for nb in (2, 3, 4, 6, 8) for ks in (1, 4)])
+def test_every_tile_and_part(bits, group, nb, parts, monkeypatch):
+    """Every kernel, on batches of exactly one tile and of two with a last row alone, raw and transformed."""
+    if group < 32 and (parts == 4 or nb in (3, 6)):
+        pytest.skip("groups of 8 and 16 have tiles of 2, 4 and 8 rows in one part")
+    monkeypatch.setenv("NEEDLE2_GPU_FP32_BATCH", f"{nb},{parts}")
+    for dim in (2100, 500) if group <= 64 else (2100,):
+        packed, norms, cb, dense = example(bits, rows=270, dim=dim, group=group, seed=group + nb + dim)
+        q = CQMatrix(packed, norms, dense.shape, bits, group, cb)
+        for batch in (nb, 2 * nb + 1):
+            x = activations((batch, dim), seed=batch)
+            expected = oracle.cq_linear(packed, norms, dense.shape, bits, group, cb, x, 4)
+            np.testing.assert_array_equal(q.matvec(x), expected)
+
+
+@pytest.mark.parametrize("group", [128, 256])
+def test_two_rows_of_many_tiles(group):
+    """Two 4-bit rows over 33 row tiles of 2100 columns, which take the batch kernel by themselves."""
+    packed, norms, cb, dense = example(4, rows=8200, dim=2100, group=group, seed=group)
+    x = activations((2, 2100), seed=3)
+    q = CQMatrix(packed, norms, dense.shape, 4, group, cb)
+    np.testing.assert_array_equal(q.matvec(x), oracle.cq_linear(packed, norms, dense.shape, 4, group, cb, x, 8))
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
@@ -104,8 +130,9 @@ def test_first_call_in_a_capture(group):
 
 @pytest.mark.parametrize("group", [32, 128])
 def test_more_rows_than_a_grid_holds(group):
-    """70000 rows: past the 65535 blocks of a grid's y, one row per pass over the codes in one launch."""
+    """70001 rows: past the 65535 blocks of a grid's y, the one-row kernels in one launch (groups up to 64: rows in
+    pairs, the last alone)."""
     packed, norms, cb, dense = example(4, rows=3, dim=128, group=group, seed=group)
-    x = activations((70000, 128), seed=1)
+    x = activations((70001, 128), seed=1)
     q = CQMatrix(packed, norms, dense.shape, 4, group, cb)
     np.testing.assert_array_equal(q.matvec(x), oracle.cq_linear(packed, norms, dense.shape, 4, group, cb, x, 8))

@@ -96,9 +96,10 @@ def test_small_groups_with_and_without_prepass(bits, group, dim, monkeypatch):
 @pytest.mark.parametrize("batch", [2, 3, 5])
 @pytest.mark.parametrize("dim", [300, 1000])
 def test_batched_rows_in_pairs(group, batch, dim, monkeypatch):
-    """4-bit batches of two or more rows take two rows per pass over the codes (cq_gemv_quad_pair_kernel: the
-    chunks loaded once for both rows' tables, an odd last row alone), for raw inputs (<= 512 wide) and the
-    pre-pass; bit-identical to the oracle and to one row per pass (NEEDLE2_GPU_FP32_PAIRS=never)."""
+    """4-bit batches of two rows take both per pass over the codes (cq_gemv_quad_pair_kernel: the chunks loaded
+    once for both rows' tables), larger ones the batch kernel (an odd last row of the pair kernel:
+    test_more_rows_than_a_grid_holds), for raw inputs (<= 512 wide) and the pre-pass; bit-identical to the oracle
+    and to one row per pass (NEEDLE2_GPU_FP32_PAIRS=never)."""
     packed, norms, cb, dense = example(4, rows=300, dim=dim, group=group, seed=31 * group + batch)
     x = activations((batch, dim), seed=group + batch)
     expected = oracle.cq_linear(packed, norms, dense.shape, 4, group, cb, x, 4)

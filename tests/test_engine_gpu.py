@@ -270,6 +270,22 @@ def test_prefill_equals_steps(window, long):
     np.testing.assert_array_equal(e3.prefill(prompt, last_only=True)[0], np.stack([e4.step(t)[0] for t in prompt])[-1])
 
 
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("window", [0, 256])
+def test_long_prefill_equals_steps_in_groups_of_128(bits, window):
+    """Chunks above 128 tokens run the transform and the batch kernel over all of a chunk's tokens, with each
+    matrix's rows strided in its layer's buffers: in the released model's groups (128) and hidden width (512), bit
+    for bit the steps' results. 300 tokens (chunks of 256 and 44) and 129 (the shortest such chunk)."""
+    geometry = dict(HEADS128, d_model=512, hada_n=512, engram_sub_dim=128, max_seq_len=512)
+    a = Archive(synthetic_model(geometry, engram_layers=(1,), engram_orders=(2, 3), kv_window=window, group=128, seed=17,
+                                layer_bits=bits))
+    for prompt in (LONG_PROMPT, LONG_PROMPT[:129]):
+        e1, e2 = GpuEngine(a), GpuEngine(a)
+        stepped = np.stack([e1.step(t)[0] for t in prompt])
+        np.testing.assert_array_equal(e2.prefill(prompt)[0], stepped)
+        np.testing.assert_array_equal(e2.step(4)[0], e1.step(4)[0])
+
+
 # G * head_dim = 128: the out-projection's groups of 128 positions are one kv head's query heads
 HEADS128 = dict(SMALL, num_heads=4, num_kv_heads=2, head_dim=64)
 
