@@ -63,6 +63,10 @@ def lib():
     return L
 
 
+class RefAbsent(RuntimeError):
+    """A call of the reference's own code where its library was not built (tests/conftest.py skips such tests)."""
+
+
 @functools.lru_cache(maxsize=1)
 def ref():
     path = HERE / "_ref" / "libref.so"
@@ -225,7 +229,7 @@ class RefCQ:
     def __init__(self, packed, norms, shape, bits, group, cb):
         L = ref()
         if L is None:
-            raise RuntimeError("oracle/_ref was not built (reference sources absent)")
+            raise RefAbsent("oracle/_ref was not built (reference sources absent)")
         self.L = L
         self.shape = tuple(shape)
         self.bits, self.group = bits, group
@@ -300,7 +304,7 @@ class RefAttention:
     def __init__(self, heads, kvheads, head_dim, max_seq, threads=1):
         L = ref()
         if L is None:
-            raise RuntimeError("oracle/_ref was not built (reference sources absent)")
+            raise RefAbsent("oracle/_ref was not built (reference sources absent)")
         self.L = L
         self.heads, self.kvheads, self.hd = heads, kvheads, head_dim
         self.h = L.refh_attn_create(heads, kvheads, head_dim, max_seq, threads)
@@ -340,7 +344,7 @@ def RefEngine(archive, activation_bits=0, int8_kv=False, threads=1, sdot=False):
     from openneedle_amd.engine import EngineBinding
     L = ref()
     if L is None:
-        raise RuntimeError("oracle/_ref was not built (reference sources absent)")
+        raise RefAbsent("oracle/_ref was not built (reference sources absent)")
     eng = EngineBinding(L, archive, RefCQ.from_record, activation_bits, threads)
     if sdot:  # the Engine's int8 matmul path (engine.cpp:424-432 without the ARM feature test)
         L.refh_engine_sdot.argtypes, L.refh_engine_sdot.restype = [ct.c_void_p], ct.c_int
