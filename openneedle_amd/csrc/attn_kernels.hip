@@ -516,6 +516,19 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
     const bool store_here =
         a.new_k && ns >= 0 && static_cast<uint32_t>(ns) < cap && sp == min(ns / a.slots_per_split, a.splits - 1);
     const bool store_early = store_here && ns < begin + 256;  // the slot may be in a first sub-tile
+    // q ahead of the tile: its split then runs while the tile is on its way. Lane (head qg, four-value part qj, chunk
+    // quad) splits its four values of each chunk.
+    const int qg = col >> 2, qj = col & 3;
+    const bool qlive = qg < GQ && 4 * qj < KB;
+    const int qd = quad * (KB * KH) + 4 * qj;
+    float qx[HQ][KH][4];
+#pragma unroll
+    for (int hq = 0; hq < HQ; ++hq)
+#pragma unroll
+        for (int h = 0; h < KH; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qx[hq][h][e] = qlive ? qh[(hq * 4 + qg) * HD + qd + h * KB + e] : 0.0f;
+    asm volatile("" ::: "memory");
     Tile cur, nxt;
     int st = begin + wave * 64;
     if (store_early) store_new<HD>(a, ns, seq, kh, row0);
@@ -533,23 +546,19 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
         return *reinterpret_cast<const i32x4 *>(wd[wave][hq][g] + (col >> 2) * 80 + (col & 3) * 16 + quad * 4);
     };
 
-    // q as operand A. Lane (head qg, four-value part qj, chunk quad) splits its four values of each chunk.
-    const int qg = col >> 2, qj = col & 3;
-    const bool qlive = qg < GQ && 4 * qj < KB;
+    // q as operand A
     i32x4 q8[HQ][2][KH];
     int qe[HQ];      // of score lane's head: exponent of the first group's last digit
     bool qleft[HQ];  // wave-uniform: qrest is not all zero
     float qscale[HQ];
 #pragma unroll
     for (int hq = 0; hq < HQ; ++hq) {
-        const int d0 = quad * (KB * KH) + 4 * qj;
-        float x[KH][4];
+        float (&x)[KH][4] = qx[hq];
         uint32_t top = 0;
 #pragma unroll
         for (int h = 0; h < KH; ++h)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                x[h][e] = qlive ? qh[(hq * 4 + qg) * HD + d0 + h * KB + e] : 0.0f;
                 const uint32_t bits = __builtin_bit_cast(uint32_t, x[h][e]) & 0x7FFFFFFFu;
                 top = top > bits ? top : bits;
             }
@@ -591,7 +600,7 @@ __global__ __launch_bounds__(256, 2) void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
             for (int h = 0; h < KH; ++h)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) qrest[wave][hq][qg][d0 + h * KB + e] = x[h][e];
+                for (int e = 0; e < 4; ++e) qrest[wave][hq][qg][qd + h * KB + e] = x[h][e];
         }
     }
     lds_fence();
