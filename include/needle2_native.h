@@ -134,11 +134,12 @@ int needle2_gpu_sdot_linear_device(void *sdot_handle, const float *d_x, float *d
 
 /* The int32 group dots of the int8 product (the accumulators of SdotCQ::dot_group,
  * needle2/csrc/sdot.cpp:108-137): d_dots[b][row][g] = sum over group g of
- * centroid(code) * q(x_b), from the kernels needle2_gpu_sdot_linear_device runs
- * for this batch on a large matrix (batch 1: the row kernel; 2 .. 8: the
- * 4x4x4 batch-tile MFMA kernel; 9 or more: the 16x16x32 batch-tile MFMA
- * kernel where a group holds whole code chunks, else the 4x4x4 one). Groups
- * of 8 .. 256. */
+ * centroid(code) * q(x_b), from the kernels with int32 accumulators (batch 1:
+ * the row kernel; 2 .. 8: the 4x4x4 batch-tile MFMA kernel; 9 or more: the
+ * 16x16x32 batch-tile MFMA kernel where a group holds whole code chunks, else
+ * the 4x4x4 one). needle2_gpu_sdot_linear_device runs these too, except on
+ * small matrices (K split) and on 4-bit groups of 32 .. 128 at 2 .. 12 rows of
+ * a large one, whose kernel holds the same dots in fp32. Groups of 8 .. 256. */
 int needle2_gpu_sdot_dots_device(void *sdot_handle, const float *d_x, int32_t *d_dots, int batch, void *stream);
 
 /* No counterpart in the reference: needle2_gpu_sdot_linear_device for callers

@@ -183,9 +183,10 @@ __host__ __device__ inline size_t norm_index(int r, int g, int groups) {
 // Where the FP32 GEMV's activations are transformed. One row: groups of 128
 // and 256 inside the kernel, groups up to 64 in a pre-pass (launch_rot_many)
 // or inside the quarter-split kernel (narrow inputs). Batches: groups up to 64
-// as for one row, 128 and 256 in the pre-pass (groups of 128 transformed by
-// the batch kernel itself measured slower: a 512-token engine prompt 4.87 ->
-// 5.24 ms). Groups above one window always use the generic transform pass.
+// as for one row, 128 and 256 in the pre-pass where the batch kernel takes them
+// (groups of 128 transformed by the batch kernel itself measured slower: a
+// 512-token engine prompt 4.87 -> 5.24 ms). Groups above one window always use
+// the generic transform pass.
 inline bool gemv_fuses_fwht(int group) { return group > 64 && group <= kWindow; }
 
 // Largest group the int8 path's one-launch prepare (FWHT + quantize in LDS) takes.

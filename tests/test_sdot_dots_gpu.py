@@ -1,9 +1,11 @@
 """The int32 accumulators of the int8 path, read directly (needle2_gpu_sdot_dots_device), against the
 reference's dot_group arithmetic (sdot.cpp:108-137) as the oracle restates it (nd_sdot_dots, itself pinned
 against the integer closed form sum(clip(rint(cb / cs)) * clip(rint(rot / scale))) in tests/test_oracle.py):
-bit-exact on every (batch row, weight row, group), on the kernels the GEMV runs for the batch (batch 1: the
-row kernel; 2 .. 8: the 4 x 4 x 4 batch-tile MFMA kernel; 9 or more: the 16 x 16 x 32 batch-tile MFMA kernel
-where the group holds whole code chunks, else the 4 x 4 x 4 one)."""
+bit-exact on every (batch row, weight row, group), on the kernels with int32 accumulators (batch 1: the row
+kernel; 2 .. 8: the 4 x 4 x 4 batch-tile MFMA kernel; 9 or more: the 16 x 16 x 32 batch-tile MFMA kernel where the
+group holds whole code chunks, else the 4 x 4 x 4 one). The fp16 batch kernel, which the GEMV runs for some batches
+of large 4-bit matrices, holds the same dots in fp32 and is held to the oracle by its outputs
+(test_sdot_batch_gpu.py)."""
 import numpy as np
 import pytest
 
