@@ -313,8 +313,8 @@ void launch_sdot_quantize(const float *rot, int rot_stride, int nvec, int padded
 // The batch (uniform across jobs) is processed in tiles that decode each code once.
 void launch_sdot_gemv(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs_dev, int njobs, int total_blocks,
                       int batch, hipStream_t s);
-// sdot_batch.hip: 4-bit codes, batches of 2 and more, groups of 32 .. 1024; false, with nothing launched, for other shapes and rows
-// whose scales exceed its LDS.
+// sdot_batch.hip: 4-bit codes, 2 .. 12 rows, groups of 32 .. 128; false, with nothing launched, for other shapes and
+// rows whose scales exceed its LDS.
 bool launch_sdot_batch(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs_dev, int njobs, int total_blocks,
                        int batch, hipStream_t s);
 // As launch_sdot_gemv for the K-split kernel's shapes (small matrices, batch

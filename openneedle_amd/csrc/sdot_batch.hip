@@ -1,5 +1,5 @@
-// gfx950 int8 ("SDOT") GEMV of 4-bit codes for batches of activation rows
-// (tiles of up to 12) and groups of 32 and more:
+// gfx950 int8 ("SDOT") GEMV of 4-bit codes for 2 to 12 activation rows and
+// groups of 32, 64 and 128:
 //   value[b][row] += (float(dot_g) * (half(norm) * cs)) * x_scale[b][g]
 // for g in group order (sdot.cpp:43-44, 142-149), bit-identical to the
 // kernels of sdot_kernels.hip.
@@ -8,7 +8,7 @@
 // codes into int8 centroids, and four instructions per (weight row, batch row,
 // group), for whole quads or sixteens of batch rows. Here
 // - codes and activations are multiplied as fp16: integers up to 127 are exact
-//   there, their products and sums of up to 1024 of them exact in the fp32
+//   there, their products and sums of a group exact in the fp32
 //   accumulators, so the matrix cores deliver float(dot) itself and the
 //   epilogue is three instructions for the batch rows there are;
 // - a byte of codes is looked up as a pair of fp16 centroids, in a 256-entry
@@ -109,12 +109,12 @@ __device__ __forceinline__ void sd_for(F &&f) {
 
 template <int GROUP, int NB>
 __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, const uint32_t *table,
-                                        const float *scales, int blk, int b0) {
+                                        const float *scales, int blk) {
     using S = SdShape<GROUP, NB>;
     constexpr int NN = S::kNorms, NQ = S::kQuads, D = S::kDwords;
     const int r = threadIdx.x % kRowsPerBlock, lane = threadIdx.x & 63;
     const int tile = blk - J.block_begin;
-    const int nb = min(NB, J.batch - b0);
+    const int nb = min(NB, J.batch);
     const int dev = geom.windows * kWindow;  // activation bytes per batch row
     const __amdgpu_buffer_rsrc_t codes =
         buffer_rsrc(J.codes + static_cast<size_t>(tile) * geom.chunks * kRowsPerBlock,
@@ -122,7 +122,7 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
     const __amdgpu_buffer_rsrc_t norms = buffer_rsrc(J.norms + static_cast<size_t>(tile) * geom.groups * kRowsPerBlock,
                                                      static_cast<uint32_t>(geom.groups) * kRowsPerBlock * 2u);
     const __amdgpu_buffer_rsrc_t acts =
-        buffer_rsrc(reinterpret_cast<const int8_t *>(J.q) + static_cast<size_t>(b0) * dev, static_cast<uint32_t>(nb) * dev);
+        buffer_rsrc(J.q, static_cast<uint32_t>(nb) * dev);
     const uint32_t code_lane = r * 16u, norm_lane = r * 2u, lane4 = lane * 4u;
     const int bpg_shift = GROUP < kSdBlock ? 0 : __builtin_ctz(geom.group / kSdBlock);
     const int i4 = lane >> 2;  // the lane's positions 4 i4 .. of the block
@@ -244,7 +244,7 @@ __device__ __forceinline__ void sd_rows(const SdotJob &J, const SdotGeom &geom, 
     if (row < J.rows) {
 #pragma unroll
         for (int b = 0; b < NB; ++b)
-            if (b < nb) ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b0 + b) * ys + row] = value[b];
+            if (b < nb) ((ND_GLOBAL float *)J.y)[static_cast<size_t>(b) * ys + row] = value[b];
     }
 }
 
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kRowsPerBlock, 2) void sdot_batch_kernel(SdotJob jo
     // (a static table: its address folds into the lookups)
     __shared__ __attribute__((aligned(16))) uint32_t table[kSdPairTable];
     extern __shared__ __attribute__((aligned(16))) float scales[];  // [groups][kScaleRow]
-    const int blk = blockIdx.x, b0 = blockIdx.y * NB;
+    const int blk = blockIdx.x;
     SdotJob J = job0;
     if (njobs > 0) {
         const ND_CONST SdotJob *cj = (const ND_CONST SdotJob *)(jobs);
@@ -271,22 +271,21 @@ __global__ __launch_bounds__(kRowsPerBlock, 2) void sdot_batch_kernel(SdotJob jo
         J.ystride = cj[j].ystride;
     }
     fill_pair_table(table, geom);
-    const int nb = min(NB, J.batch - b0);
+    const int nb = min(NB, J.batch);
     for (int i = threadIdx.x; i < geom.groups * S::kScaleRow; i += kRowsPerBlock) {
         const int g = i / S::kScaleRow, b = i % S::kScaleRow;
-        scales[i] = b < nb ? J.xs[static_cast<size_t>(b0 + b) * geom.groups + g] : 0.0f;
+        scales[i] = b < nb ? J.xs[static_cast<size_t>(b) * geom.groups + g] : 0.0f;
     }
     __syncthreads();
-    sd_rows<GROUP, NB>(J, geom, table, scales, blk, b0);
+    sd_rows<GROUP, NB>(J, geom, table, scales, blk);
 }
 
 template <int GROUP, int NB>
-bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
-                     hipStream_t s) {
+bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, hipStream_t s) {
     using S = SdShape<GROUP, NB>;
     const size_t lds = static_cast<size_t>(g.groups) * S::kScaleRow * 4;
     if (lds + kSdPairTable * 4 > kSdMaxLds) return false;
-    const dim3 grid(blocks, (batch + NB - 1) / NB), block(kRowsPerBlock);
+    const dim3 grid(blocks), block(kRowsPerBlock);
     hipLaunchKernelGGL((sdot_batch_kernel<GROUP, NB>), grid, block, lds, s, job0, jobs, njobs, g);
     ND_HIP(hipGetLastError());
     return true;
@@ -295,16 +294,15 @@ bool sd_launch_shape(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs
 template <int GROUP>
 bool sd_launch_group(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                      hipStream_t s) {
-    const int tiles = (batch + 11) / 12, rows = (batch + tiles - 1) / tiles;  // batch rows of a tile, all alike
     auto go = [&](auto nb) {
-        return sd_launch_shape<GROUP, decltype(nb)::value>(g, job0, jobs, njobs, blocks, batch, s);
+        return sd_launch_shape<GROUP, decltype(nb)::value>(g, job0, jobs, njobs, blocks, s);
     };
-    if (rows <= 2) return go(std::integral_constant<int, 2>{});
-    if (rows <= 3) return go(std::integral_constant<int, 3>{});
-    if (rows <= 4) return go(std::integral_constant<int, 4>{});
-    if (rows <= 5) return go(std::integral_constant<int, 5>{});
-    if (rows <= 6) return go(std::integral_constant<int, 6>{});
-    if (rows <= 8) return go(std::integral_constant<int, 8>{});
+    if (batch <= 2) return go(std::integral_constant<int, 2>{});
+    if (batch <= 3) return go(std::integral_constant<int, 3>{});
+    if (batch <= 4) return go(std::integral_constant<int, 4>{});
+    if (batch <= 5) return go(std::integral_constant<int, 5>{});
+    if (batch <= 6) return go(std::integral_constant<int, 6>{});
+    if (batch <= 8) return go(std::integral_constant<int, 8>{});
     return go(std::integral_constant<int, 12>{});
 }
 
@@ -312,10 +310,10 @@ bool sd_launch_group(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs
 
 bool launch_sdot_batch(const SdotGeom &g, const SdotJob &job0, const SdotJob *jobs, int njobs, int blocks, int batch,
                        hipStream_t s) {
-    // sums of up to 1024 products of int8 values stay below 2^24; a tile's activations below 2^32 bytes
-    if (g.kind != kNib || g.group < 32 || g.group > 1024 || batch < 2 || g.windows > 1 << 19) return false;
+    // a group's products of int8 values sum below 2^24; the activations stay below 2^32 bytes
+    if (g.kind != kNib || g.group < 32 || g.group > 128 || batch < 2 || batch > 12 || g.windows > 1 << 19) return false;
     if (g.group == 32) return sd_launch_group<32>(g, job0, jobs, njobs, blocks, batch, s);
-    return sd_launch_group<64>(g, job0, jobs, njobs, blocks, batch, s);  // 64 .. 1024
+    return sd_launch_group<64>(g, job0, jobs, njobs, blocks, batch, s);  // 64 and 128
 }
 
 }  // namespace nd

@@ -1,8 +1,8 @@
 """The int8 batch GEMV on fp16 matrix instructions (sdot_batch.hip): bit-identical to the oracle.
 
-Every tile height (2 .. 12 rows; the next larger one with rows past the batch, and several tiles), groups of half a
-block of 64 positions, one block and several, up to the largest (1024 products of 127 x 127 in one fp32 sum), ragged
-rows and widths down to one block.
+Every tile height (2 .. 12 rows; the next larger one with rows past the batch), groups of half a block of 64 positions,
+one block and two, their largest sums, ragged rows and widths down to one block; larger batches and groups, which take
+the other kernels, beside them.
 """
 import numpy as np
 import pytest
@@ -41,10 +41,9 @@ def test_one_block(group):
     check(4, group, 257, 33, 5)
 
 
-@pytest.mark.parametrize("group", [64, 1024])
+@pytest.mark.parametrize("group", [64, 128, 1024])
 def test_largest_sums(group):
-    """Every activation and centroid of a group at the end of its range and of one sign: the sums of 1024 products
-    come closest to 2^24."""
+    """Every activation and centroid of a group at the end of its range and of one sign: the largest sums."""
     rows, dim = 40, 1024
     packed, norms, cb, dense = example(4, rows=rows, dim=dim, group=group, seed=group)
     packed[:] = 0xFF  # the largest code everywhere
