@@ -26,14 +26,13 @@
 // 473 / 813 us (rows in pairs before).
 #pragma once
 
+#include "batch_pick.h"
 #include "codes.h"
 #include "common.h"
 #include "wave.h"
 
 #include <hip/hip_fp16.h>
 
-#include <cstdio>
-#include <cstdlib>
 #include <type_traits>
 #include <utility>
 
@@ -371,45 +370,6 @@ void launch_shape(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njo
     ND_HIP(hipGetLastError());
 }
 
-struct BatchPick {
-    int nb, ks;
-};
-
-// Tile height (batch rows per workgroup) and K parts. A SIMD issues about one
-// wave instruction per 4 clocks, so a wave's cost per position is its adds,
-// its MFMAs and ~2 for the centroid lookups; below two waves per SIMD it runs
-// 1.6 times slower (27.7 against 17.4 ns, see above). Fewer rows per tile
-// repeat the lookups, more rows leave SIMDs idle; four parts divide a row's
-// walk by four where tiles alone do not fill the chip. NEEDLE2_GPU_FP32_BATCH =
-// "rows,parts" picks them, where the group has such a kernel.
-BatchPick pick(const CqGeom &g, int blocks, int batch) {
-    constexpr int kSimds = 1024;
-    auto parts_ok = [&](int ks) {
-        return ks == 1 || (g.group >= 32 && g.groups * (g.group < 64 ? g.group : 64) >= 4 * 64 && g.groups >= 4);
-    };
-    auto rows_ok = [&](int nb) { return g.group >= 32 || (nb != 3 && nb != 6); };
-    if (const char *mode = std::getenv("NEEDLE2_GPU_FP32_BATCH")) {
-        int nb = 0, ks = 0;
-        if (std::sscanf(mode, "%d,%d", &nb, &ks) == 2 && (ks == 1 || ks == 4) && parts_ok(ks) &&
-            (nb == 2 || nb == 3 || nb == 4 || nb == 6 || nb == 8) && rows_ok(nb))
-            return {nb, ks};
-    }
-    BatchPick best{2, 1};
-    double cost = 0;
-    for (int ks : {1, 4}) {
-        if (!parts_ok(ks)) continue;
-        for (int nb : {2, 3, 4, 6, 8}) {
-            if (!rows_ok(nb)) continue;
-            const double waves = 4.0 * ks * blocks * ((batch + nb - 1) / nb);
-            const double per_simd = waves / kSimds;
-            const double turns = per_simd <= 1 ? 1.6 : per_simd <= 2 ? 2 : per_simd;
-            const double c = turns * (nb + (nb + 3) / 4 + 2.0) / ks * (ks > 1 ? 1.05 : 1.0);
-            if (cost == 0 || c < cost) cost = c, best = {nb, ks};
-        }
-    }
-    return best;
-}
-
 template <int KIND, int GROUP, int NB>
 void launch_parts(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, int batch, bool x_raw,
                   int ks, hipStream_t s) {
@@ -422,7 +382,7 @@ void launch_parts(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njo
 template <int KIND, int GROUP>
 void launch_group(const CqGeom &g, const CqJob &job0, const CqJob *jobs, int njobs, int blocks, int batch, bool x_raw,
                   hipStream_t s) {
-    const BatchPick b = pick(g, blocks, batch);
+    const BatchPick b = batch_pick(g.kind, g.group, g.groups, blocks, batch);
     if constexpr (GROUP >= 32) {
         if (b.nb == 3) return launch_parts<KIND, GROUP, 3>(g, job0, jobs, njobs, blocks, batch, x_raw, b.ks, s);
         if (b.nb == 6) return launch_parts<KIND, GROUP, 6>(g, job0, jobs, njobs, blocks, batch, x_raw, b.ks, s);

@@ -7,6 +7,7 @@
 // rebuilt per 256-position window and shared by the workgroup's 256 rows, so
 // each code costs one LDS read plus one add, in the reference's own order.
 // All files are compiled with -ffp-contract=off.
+#include "batch_pick.h"
 #include "codes.h"
 #include "common.h"
 #include "wave.h"
@@ -1473,27 +1474,36 @@ static bool gemv_quad_takes_x(int group, int in) {
 
 // Whether the batch kernel pays against one row per pass (two 4-bit rows of
 // groups up to 64: the pair kernel). Groups of 128 and 256 then need the
-// pre-pass that one row per pass does without, some 3 us, so their line lies
-// where the rows' walks cost more: `walk` counts windows walked again after the
-// first row, groups of 256 (whose one-row walk takes twice as long) twice.
-// Plans of 32 and more row tiles, one row per pass against the batch kernel:
-// CQ4 g128, 2 rows, 512 / 1100 / 2048 columns 8.9 / 20.3 / 30.3 against 11.3 /
-// 22.6 / 28.0 us, 3 rows, 256 / 512 8.7 / 12.2 against 10.2 / 11.5; CQ4 g256, 2
-// rows, 768 / 1100 18.8 / 29.4 against 19.5 / 27.7; CQ2 g128, 3 rows, 768 / 1100
-// 15.9 / 24.2 against 18.1 / 23.1, 4 rows, 512 / 768 12.1 / 20.4 against 13.2 /
-// 18.1; CQ2 g256, 3 rows, 512 / 1100 14.2 / 30.4 against 15.5 / 28.0. Other
+// pre-pass that one row per pass does without, some 3 us, so both ways are
+// priced, in us of a call among others: one row per pass by the windows walked,
+// more once the row tiles outnumber the CUs, the batch kernel by its pick. Fitted
+// to 1372 shapes (16 to 512 row tiles, 256 to 2048 columns, 2 to 8 rows): the
+// slower way is taken by more than 6% in 25 of them, at most 15%. E.g. CQ4 g128,
+// 2 rows, 512 / 1500 columns x 128 tiles 9.6 / 25.7 against 12.0 / 23.8 us, 3
+// rows, 256 / 512 8.7 / 12.2 against 10.2 / 11.5; CQ2 g128, 3 rows, 768 / 1000 15.9 /
+// 22.5 against 18.1 / 19.8, 6 rows x 256 tiles, 400 / 1000 18.5 / 42.1 against 20.6 /
+// 31.8; CQ2 g256, 3 rows, 512 / 1100 14.2 / 30.4 against 15.5 / 28.0. Other
 // groups, whose rows are transformed ahead either way: from four rows on, and
 // from three except for 2-bit groups of up to 64 (8 x 2048 x 4000: 52.0 against
 // 50.5 us one row per pass; CQ4 g32 57.8 against 72.0 in pairs); two rows only
 // of 4-bit groups above 256 and from 32 row tiles on (CQ4 g32 52.0 against 48.8,
 // CQ2 g64 47.8 against 35.8).
-// NEEDLE2_GPU_FP32_BATCH, the kernel's own override (cq_batch.h), takes every batch of two and more.
+// NEEDLE2_GPU_FP32_BATCH, the kernel's own override (batch_pick.h), takes every
+// batch of two and more.
 static bool batch_pays(int kind, int group, int in, int blocks, int batch) {
-    if (std::getenv("NEEDLE2_GPU_FP32_BATCH")) return batch >= 2;
+    if (batch < 2) return false;
+    if (std::getenv("NEEDLE2_GPU_FP32_BATCH")) return true;
     if (gemv_fuses_fwht(group)) {
-        const long walk = static_cast<long>(batch - 1) * ((in + kWindow - 1) / kWindow) * (group / 128);
-        if (kind == kCrumb) return batch >= 6 || (batch >= 3 && walk >= 9);
-        return batch >= 4 || (batch == 3 && walk >= 4) || (batch == 2 && walk >= 8 && blocks >= 32);
+        struct Price {
+            double call, window, more;  // one row per pass; more: a window's share per further tile on a CU
+        };
+        const Price p = kind == kNib ? (group == 128 ? Price{3.7, 1.8, 0.8} : Price{4.3, 2.56, 0.4})
+                                     : (group == 128 ? Price{2.9, 1.5, 0.6} : Price{3.9, 1.8, 0.4});
+        const int deep = (blocks + device_cus() - 1) / device_cus();
+        const double windows = static_cast<double>(batch) * ((in + kWindow - 1) / kWindow);
+        const double one = p.call + p.window * windows * (1 + p.more * (deep - 1));
+        const double cost = batch_pick(kind, group, (in + group - 1) / group, blocks, batch).cost;
+        return (kind == kNib ? 6.55 + 0.138 * cost : 8.45 + 0.1275 * cost) < one;
     }
     return batch >= 4 || (batch == 3 && !(kind == kCrumb && group <= 64)) ||
            (batch == 2 && kind == kNib && group > 64 && blocks >= 32);
